@@ -1,51 +1,62 @@
-"""Build-time check of the prefill kernel's inline-asm MFMAs.
+"""Build-time checks of the prefill kernels' inline-asm MFMAs.
 
 `prefill_mfma_kernel` issues its PV MFMAs as inline asm (so that the O^T
-accumulators stay in AGPRs).  The compiler cannot see an MFMA inside asm, so
-it neither inserts the wait states the MFMA's result needs before another
-instruction reads it nor avoids placing a register copy of the accumulator
-right after it.  If it ever places such a copy, the copy reads the
-accumulator before the MFMA has written it and the results are wrong
-(a code change that let this happen computed wrong prefill outputs).  The
-build therefore scans the kernel's gfx950 assembly and fails on any read of
-an inline-asm MFMA's destination AGPRs within the MFMA's result latency.
+accumulators stay in AGPRs), `prefill_wide_kernel` all of its MFMAs.  The
+compiler cannot see an MFMA inside asm, so it neither inserts the wait states
+the MFMA needs around it nor avoids placing a register copy right behind it.
+The build therefore scans the kernels' gfx950 assembly and fails on
+
+* any read of an inline-asm MFMA's destination registers, or (vector registers)
+  any write to them, within the MFMA's result latency: a copy of an accumulator
+  placed there once computed wrong prefill outputs;
+* any vector instruction that writes an operand of an inline-asm MFMA within
+  the two wait states before it;
+* in kernels that address the accumulation registers by number (`owned_agprs`),
+  any use of one outside asm: it would overwrite an accumulator.
 """
 from __future__ import annotations
 
 import re
 
 # Wait states a v_mfma_f32_32x32x16_bf16 result (16 passes) needs before a
-# VALU or v_accvgpr read of it; the kernel's own drain after each tile's PV
-# batch gives 20 (s_nop 7, s_nop 7, s_nop 3).
+# VALU or v_accvgpr read of it; the kernels' drains give 20 (s_nop 7, s_nop 7,
+# s_nop 3).
 RESULT_WAIT_STATES = 19
+# Wait states between a VALU write of a register and an MFMA that reads it.
+OPERAND_WAIT_STATES = 2
 
-_AGPR_RANGE = re.compile(r"^a\[(\d+):(\d+)\]$")
-_AGPR_ONE = re.compile(r"^a(\d+)$")
+_INDEX = r"(0x[0-9a-f]+|\d+)"
+_REGISTER = re.compile(rf"\b([av])\[{_INDEX}:{_INDEX}\]|\b([av])\[?{_INDEX}\b")
 _NOP = re.compile(r"^s_nop\s+(\d+)")
 
 
-def _agprs(operand: str):
-    operand = operand.strip()
-    m = _AGPR_RANGE.match(operand)
-    if m:
-        return int(m.group(1)), int(m.group(2))
-    m = _AGPR_ONE.match(operand)
-    if m:
-        return int(m.group(1)), int(m.group(1))
-    return None
+def _registers(operand: str):
+    """(file, first, last) of every vector / accumulation register named."""
+    found = []
+    for m in _REGISTER.finditer(operand):
+        if m.group(1):
+            found.append((m.group(1), int(m.group(2), 0), int(m.group(3), 0)))
+        else:
+            found.append((m.group(4), int(m.group(5), 0), int(m.group(5), 0)))
+    return found
 
 
-def asm_mfma_hazards(assembly: str) -> list[str]:
-    """Reads of an inline-asm MFMA's destination AGPRs issued fewer than
-    RESULT_WAIT_STATES wait states after it (s_nop n counts n + 1, any other
-    instruction 1).  Code is followed in listing order, labels included, so a
-    fall-through is checked like straight-line code; a taken branch is not
-    followed (the kernel drains its asm MFMAs before each loop back-edge).
-    Reads by other MFMAs are not checked: the kernel's accumulators feed only
-    the next MFMA of their own chain, which the hardware's dependency check
-    covers."""
+def _overlap(x, y) -> bool:
+    return x[0] == y[0] and x[1] <= y[2] and y[1] <= x[2]
+
+
+def asm_mfma_hazards(assembly: str, owned_agprs: bool = False) -> list[str]:
+    """The violations of the rules above (s_nop n counts n + 1 wait states, any
+    other instruction 1).  Code is followed in listing order, labels included,
+    so a fall-through is checked like straight-line code; a taken branch is not
+    followed (prefill_mfma_kernel drains its asm MFMAs before each loop
+    back-edge, prefill_wide_kernel has the next tile's first operand reads and
+    the max of its scores there).  Reads by other MFMAs are not checked: an
+    accumulator feeds only the next MFMA of its own chain, which the hardware's
+    dependency check covers."""
     hazards: list[str] = []
-    pending: list[list[int]] = []  # [first AGPR, last AGPR, wait states left, line]
+    pending: list[list] = []  # [destination, wait states left, line] of asm MFMAs
+    written: list[list] = []  # [register, wait states left, line] of VALU writes
     in_asm = False
     for number, raw in enumerate(assembly.splitlines(), 1):
         text = raw.strip()
@@ -55,29 +66,41 @@ def asm_mfma_hazards(assembly: str) -> list[str]:
         if text.startswith(";;#ASMEND"):
             in_asm = False
             continue
-        if not text or text.startswith((";", ".")) or text.endswith(":"):
+        text = text.split(";")[0].strip()
+        if not text or text.startswith(".") or text.endswith(":"):
             continue
+        issued = None  # the destination of an asm MFMA on this line
         opcode = text.split()[0]
-        operands = [x for x in text[len(opcode):].split(",")]
+        operands = [_registers(x) for x in text[len(opcode):].split(",")]
         nop = _NOP.match(text)
         if opcode.startswith("v_mfma"):
-            if in_asm:
-                dest = _agprs(operands[0])
-                if dest is not None:
-                    pending.append([dest[0], dest[1], RESULT_WAIT_STATES, number])
-                    continue
+            if in_asm and operands[0]:
+                for source in operands[1] + operands[2]:
+                    for register, left, line in written:
+                        if left > 0 and _overlap(register, source):
+                            hazards.append(f"line {number}: '{text}' reads a register written at line {line}, "
+                                           f"{OPERAND_WAIT_STATES - left} wait states before")
+                issued = operands[0][0]
         elif nop is None:
-            for operand in operands[1:]:
-                src = _agprs(operand)
-                if src is None:
-                    continue
-                for first, last, left, line in pending:
-                    if left > 0 and not (src[1] < first or src[0] > last):
-                        hazards.append(f"line {number}: '{text}' reads a[{first}:{last}], written by the "
-                                       f"inline-asm MFMA at line {line}, after "
-                                       f"{RESULT_WAIT_STATES - left} wait states")
+            stores = opcode.startswith("ds_write") or "store" in opcode
+            reads = [r for x in (operands if stores else operands[1:]) for r in x]
+            writes = [r for r in operands[0] if r[0] == "v"] if opcode.startswith("v_") else []
+            for verb, registers in (("reads", reads), ("writes", writes)):
+                for register in registers:
+                    for dest, left, line in pending:
+                        if left > 0 and _overlap(dest, register):
+                            hazards.append(f"line {number}: '{text}' {verb} {dest[0]}[{dest[1]}:{dest[2]}], written by "
+                                           f"the inline-asm MFMA at line {line}, after "
+                                           f"{RESULT_WAIT_STATES - left} wait states")
+            if owned_agprs and not in_asm and any(r[0] == "a" for x in operands for r in x):
+                hazards.append(f"line {number}: '{text}' uses an accumulation register outside asm")
         step = int(nop.group(1)) + 1 if nop else 1
-        for entry in pending:
-            entry[2] -= step
-        pending = [entry for entry in pending if entry[2] > 0]
+        for entry in pending + written:
+            entry[1] -= step
+        pending = [e for e in pending if e[1] > 0]
+        if issued is not None:
+            pending.append([issued, RESULT_WAIT_STATES, number])
+        written = [e for e in written if e[1] > 0]
+        if opcode.startswith("v_") and not opcode.startswith("v_mfma") and operands[0]:
+            written.append([operands[0][0], OPERAND_WAIT_STATES, number])
     return hazards

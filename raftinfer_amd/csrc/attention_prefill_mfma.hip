@@ -1,5 +1,6 @@
 // Causal gated GQA prefill attention for the Qwen3.5 signature (16 query
-// heads, 4 KV heads, head_dim 256) on gfx950 bf16 MFMA.
+// heads, 4 KV heads, head_dim 256) on gfx950 bf16 MFMA, for short prompts and
+// short pasts (prefill_plan; attention_prefill_wide.hip takes the others).
 //
 // Work split.  A workgroup owns one KV head and 8 query tokens.  The 4 query
 // heads of the GQA group x the 8 tokens are the 32 columns of one MFMA
@@ -37,23 +38,16 @@
 // neither goes out as scattered 8-byte pieces and only one barrier follows
 // the loop.  With past == 0 the keys come from the key/value
 // inputs and each workgroup also writes its 8 tokens' cache rows (the append).
-#include "decode_scan.hpp"
-#include "norm_rope.hpp"
 #include "prefill_mfma.hpp"
+#include "prefill_tile.hpp"
 
 namespace raftinfer::amd {
 namespace {
 
-constexpr int kQTok = 8;             // query tokens per workgroup
-constexpr int kKTile = 32;           // keys per tile
-constexpr int kWaves = 4;            // key-split waves per workgroup
-constexpr int kThreads = kWaves * kWave;
-constexpr float kLazyRescale = 8.0f; // log2 units
-constexpr int kPvBatch = 8;          // PV MFMAs whose operands are read together
-constexpr int kHalfElems = kKTile * kHeadDim / 2; // one half of a K / V tile (128 dims)
+using namespace prefill;
 
-typedef short short4v __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) short4v lds_short4v;
+constexpr int kQTok = 8;    // query tokens per workgroup
+constexpr int kPvBatch = 8; // PV MFMAs whose operands are read together
 
 struct WaveTile {
   bf16_bits k[kKTile * kHeadDim];
@@ -71,119 +65,10 @@ struct PrefillShared {
   float l[kWaves][kWave];
 };
 
-// The q producer fused into the prefill kernel (NormQ).
-struct PrefillNormRope {
-  const void *weight; // q norm weight [256], bf16 or f32
-  bool weight_f32;
-  int pairs;    // rotary_dim / 2 (rotary_dim a multiple of 8)
-  double ratio; // rope_base^(-2 / rotary_dim)
-  float epsilon;
-};
 struct alignas(16) NormQShared {
   float weight[kHeadDim];        // the staged norm weight (bf16 uses the first half)
   float rot[kQTok][kHeadDim];    // per token slot: cos[pairs] then sin[pairs]
 };
-
-// Physical 16-byte chunk of logical chunk c in tile row r: c ^ (r & 7).  The
-// LDS bank-conflict counter, calibrated on these access patterns alone, shows
-// this leaves 2-way conflicts on the K/Q ds_read_b128 (16 rows per pass) and
-// 4-way on the V ds_read_b64_tr_b16; c ^ (4 (r % 4) + (r / 4) % 4) is free of
-// both, but measured PP512 13.2 -> 13.1 us, PP2048 80 -> 78, PP128 7.13 ->
-// 7.3 (more lane bases held across the loop), so the loop is not bound by
-// these reads and the simpler swizzle stays.
-__device__ __forceinline__ int swz(int r) { return r & 7; }
-
-__device__ __forceinline__ int chunk_offset(int r, int c) { // in bf16 elements
-  return r * kHeadDim + ((c ^ swz(r)) << 3);
-}
-
-__device__ __forceinline__ bf16x8 lds_b128(const bf16_bits *p) {
-  return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(p));
-}
-
-__device__ __forceinline__ u32x2 lds_tr16(const bf16_bits *p) {
-  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v *)(p)));
-}
-
-
-
-__host__ __device__ constexpr std::size_t ceil_div_u(std::size_t n, std::size_t d) {
-  return (n + d - 1) / d;
-}
-
-// o += a * b (v_mfma_f32_32x32x16_bf16) with the accumulator pinned to AGPRs.
-// The compiler would otherwise move all 128 accumulator registers between
-// AGPRs and VGPRs around every tile because of the (rare) rescale code.  The
-// s_nop covers the VALU-write -> MFMA-read hazard of the operands, which the
-// hazard recognizer does not see through asm.  For the same reason the
-// compiler does not know the MFMA's result latency: a register copy of `o`
-// placed right after this statement would read it before it is written.  The
-// build (raftinfer_amd/asm_check.py) scans this file's assembly and fails on
-// any such read; the drain below covers the reads the kernel itself makes.
-__device__ __forceinline__ void mfma_acc_agpr(floatx16 &o, bf16x8 a, bf16x8 b) {
-  asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(o) : "v"(a), "v"(b));
-}
-// o *= s for an AGPR-resident accumulator.  The empty asm statements pin the
-// copy to VGPRs inside this (rare) rescale path; without them the compiler
-// hoists the AGPR -> VGPR copies of all accumulators onto every tile.
-__device__ __forceinline__ void scale_agpr(floatx16 &o, float s) {
-  floatx16 x = o;
-  asm volatile("" : "+v"(x));
-#pragma unroll
-  for (int i = 0; i < 16; ++i) x[i] *= s;
-  asm volatile("" : "+v"(x));
-  o = x;
-}
-// Wait states after the last such MFMA before VALU code reads its result.
-__device__ __forceinline__ void mfma_drain() { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" ::: "memory"); }
-
-__device__ __forceinline__ float fexp2(float x) { return __builtin_amdgcn_exp2f(x); }
-
-// The q producer's RMSNorm + RoPE applied in place to the staged Q rows, bit
-// for bit.  Sliced form (rotary pairs a multiple of 32; norm_rope_256_slice):
-// eight lanes per row, so a wave finishes its 8 rows at once with one LDS
-// round trip.
-__device__ __forceinline__ void norm_rope_rows_sliced(bf16_bits *q, int r, int g, const float *weight,
-                                                      bool weight_f32, int pairs, const float *rot,
-                                                      float epsilon) {
-  bf16_bits *row = q + r * kHeadDim;
-  u32x4 raw[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const u32x4 *>(row + (((4 * g + j) ^ swz(r)) << 3));
-  float x[32], w[32], v[32];
-  unpack_bf16x32(raw, x);
-  load_slice_weights(weight, weight_f32, g, w);
-  norm_rope_256_slice(x, w, g, pairs, rot, epsilon, v);
-  u32x4 out[4];
-  pack_bf16x32(v, out);
-#pragma unroll
-  for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4 *>(row + (((4 * g + j) ^ swz(r)) << 3)) = out[j];
-}
-
-// Lane-wise form (any rotary width): rows 8w .. 8w+7 one at a time, lane l
-// owning dims 4l .. 4l+3 (8 bytes of logical chunk l / 2).
-__device__ __forceinline__ void norm_rope_rows_lanewise(bf16_bits *q, int wave, int lane, const float *weight,
-                                                        bool weight_f32, int pairs, const float (*rot)[kHeadDim],
-                                                        float epsilon) {
-  float w[4];
-  if (weight_f32) {
-    const float4 x = reinterpret_cast<const float4 *>(weight)[lane];
-    w[0] = x.x; w[1] = x.y; w[2] = x.z; w[3] = x.w;
-  } else {
-    const u32x2 x = reinterpret_cast<const u32x2 *>(weight)[lane];
-    w[0] = bf16_lo(x[0]); w[1] = bf16_hi(x[0]); w[2] = bf16_lo(x[1]); w[3] = bf16_hi(x[1]);
-  }
-#pragma unroll
-  for (int rr = 0; rr < 8; ++rr) {
-    const int r = 8 * wave + rr;
-    u32x2 *slot = reinterpret_cast<u32x2 *>(q + chunk_offset(r, lane >> 1) + 4 * (lane & 1));
-    const u32x2 raw = *slot;
-    const float x[4] = {bf16_lo(raw[0]), bf16_hi(raw[0]), bf16_lo(raw[1]), bf16_hi(raw[1])};
-    float v[4];
-    norm_rope_256_lane(x, w, lane, pairs, rot[r & (kQTok - 1)], epsilon, v);
-    *slot = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-  }
-}
 
 // FromInput: past == 0 and every key is read from the key/value inputs
 // ([tokens][4][256]); the workgroup also writes its own tokens' rows into the
@@ -396,7 +281,7 @@ __global__ __launch_bounds__(kThreads) void prefill_mfma_kernel(
       norm_rope_rows_sliced(sh.q, 8 * wave_u + (lane >> 3), lane & 7, nqs->weight, nq.weight_f32, nq.pairs,
                             nqs->rot[(lane >> 3) & (kQTok - 1)], nq.epsilon);
     else
-      norm_rope_rows_lanewise(sh.q, wave_u, lane, nqs->weight, nq.weight_f32, nq.pairs, nqs->rot, nq.epsilon);
+      norm_rope_rows_lanewise(sh.q, 8 * wave_u, lane, nqs->weight, nq.weight_f32, nq.pairs, nqs->rot, nq.epsilon);
     __syncthreads(); // every row is normalised
   }
   for (; t < n_tiles; t += kWaves) {
@@ -652,10 +537,35 @@ __global__ __launch_bounds__(kThreads) void prefill_mfma_kernel(
 
 } // namespace
 
+// A form with t tokens per workgroup has 4 ceil(tokens / t) workgroups, one per
+// CU at a time, and t keys' worth of work per key loaded: the larger t is the
+// faster the longer the key range, as long as the workgroups fill the 256 CUs.
+// So the lines lie where the workgroups of a form come to 256 (512, 1024, 2048
+// tokens), and below them where the longer start and end of the streaming
+// kernel is made up for.  Measured (us; short8 / stream8 / stream16 / stream32,
+// tokens behind past keys): 512 behind 0: 12.9 / 15.4 / 21 / 30, behind 512:
+// 23.5 / 23.2 / 32 / 44, behind 1024: 29.8 / 28.0 / 38 / 55; 64 behind 1024:
+// 21.2 / 19.5 / 28 / 44; 768 behind 0: 18.6 / 22 / 26 / 37, behind 1000: 49 /
+// 46 / 43 / 63; 1100 behind 0: 33 / 35 / 30 / 46; 2048 behind 0: 77 / 79 / 60 /
+// 69, behind 4000: 296 / 249 / 186 / 184; 2560 behind 0: 124 / 105 / 92 / 83;
+// 5000 behind 4000: 829 / 720 / 549 / 525.
+PrefillForm prefill_plan(std::size_t tokens, std::size_t past) {
+  if (tokens > 2048) return PrefillForm::stream32;
+  if (tokens > 1024) return PrefillForm::stream16;
+  if (tokens > 512) return past > 512 ? PrefillForm::stream16 : PrefillForm::short8;
+  return past + tokens >= 1024 ? PrefillForm::stream8 : PrefillForm::short8;
+}
+
 void launch_prefill_mfma(const bf16_bits *q, const bf16_bits *key, const bf16_bits *value,
                          const bf16_bits *gate, bf16_bits *out, bf16_bits *cache,
                          std::size_t tokens, std::size_t max_ctx, std::size_t past,
                          bool head_major, bool fused_append, hipStream_t stream) {
+  const PrefillForm form = prefill_plan(tokens, past);
+  if (form != PrefillForm::short8) {
+    launch_prefill_wide(form, q, key, value, gate, out, cache, tokens, max_ctx, past, head_major, fused_append, nullptr,
+                        stream);
+    return;
+  }
   // 8 workgroups (one per XCD) per pair of query tiles.
   const unsigned grid = static_cast<unsigned>(8 * ceil_div_unchecked(ceil_div_unchecked(tokens, kQTok), 2));
   const PrefillNormRope none{};
@@ -724,6 +634,12 @@ void launch_prefill_mfma_fused(const bf16_bits *query_gate, const bf16_bits *key
       key, value, k_weight, weight_f32, pairs, ratio, epsilon, cache, max_ctx, past, head_major);
   const unsigned grid = static_cast<unsigned>(8 * ceil_div_unchecked(ceil_div_unchecked(tokens, kQTok), 2));
   const PrefillNormRope nq{q_weight, weight_f32, pairs, ratio, epsilon};
+  const PrefillForm form = prefill_plan(tokens, past);
+  if (form != PrefillForm::short8) {
+    launch_prefill_wide(form, query_gate, nullptr, nullptr, nullptr, out, cache, tokens, max_ctx, past, head_major, false,
+                        &nq, stream);
+    return;
+  }
   if (head_major)
     prefill_mfma_kernel<true, false, true><<<grid, kThreads, 0, stream>>>(
         query_gate, key, value, nullptr, out, cache, tokens, max_ctx, past, nq);

@@ -1,0 +1,856 @@
+// Causal gated GQA prefill attention for long key ranges (gfx950 bf16 MFMA, the
+// Qwen3.5 signature): the same arithmetic as prefill_mfma_kernel on a schedule
+// that keeps the matrix units busy.
+//
+// prefill_mfma_kernel runs each wave's tile as a chain (wait, QK^T, softmax, PV)
+// at one wave per SIMD, so the matrix units idle through the softmax and through
+// most of the loads: 1.75 us per round of four 32-key tiles, where the MFMAs of
+// its 32 columns take 0.5.  Here
+//   - a wave holds NB = 1 or 2 blocks of 32 columns (4 heads x 8 tokens), so a K
+//     or V operand read from LDS feeds NB MFMAs, with the Q operands in registers
+//     and the O^T accumulators in the accumulation registers by number;
+//   - S(n + 1) = K Q^T runs on the matrix unit while the vector unit turns S(n)
+//     into probabilities, and the rest of them and the max of S(n + 1) are formed
+//     behind the MFMAs of PV(n).  One wave issues at most an instruction every
+//     four clocks, so the instructions around the MFMAs are counted: loads set
+//     their LDS address once each and take their row from the instruction's
+//     offset, operand addresses of a pair of steps share an exclusive-or;
+//   - K and V tiles stream through a ring of five LDS slots per key group, loaded
+//     by LDS-direct loads three or four ring items ahead, one load behind each
+//     MFMA group;
+//   - KS = 4 key groups: each wave streams its own 32-key tiles (no barriers in
+//     the loop); KS = 2: two waves with 64 columns each share a group's tiles,
+//     which halves the bytes and LDS writes per column for one barrier per item.
+//     Barriers and loads bound NB = 1 (128 KiB per round of 4 tiles: 1.4 us),
+//     the card's power NB = 2 (2048 tokens behind 30000: 1.2 PFLOP/s, the rate
+//     that a bf16 matrix product of 8192^3 reaches here).
+// prefill_plan (attention_prefill_mfma.hip) says which form takes a call.
+#include "prefill_mfma.hpp"
+#include "prefill_tile.hpp"
+
+#include <utility>
+
+namespace raftinfer::amd {
+namespace {
+
+using namespace prefill;
+
+__device__ __forceinline__ bf16x8 lds_read_b128(unsigned addr) {
+  return __builtin_bit_cast(bf16x8, *(const __attribute__((address_space(3))) u32x4 *)(std::uintptr_t)(addr));
+}
+__device__ __forceinline__ u32x2 lds_read_tr16(unsigned addr) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4v *)(std::uintptr_t)(addr)));
+}
+template <typename T> __device__ __forceinline__ T *lds_ptr(unsigned addr) {
+  return (T *)(__attribute__((address_space(3))) T *)(std::uintptr_t)(addr);
+}
+// off ^ x and off + a, as asm so that the results are formed where they are used:
+// hoisted out of the tile loop, the offsets of all loads took registers from the
+// Q operands.
+template <unsigned kXor, unsigned kAdd> __device__ __forceinline__ std::uint32_t load_offset(std::uint32_t off) {
+  std::uint32_t x = off;
+  if constexpr (kXor != 0) asm volatile("v_xor_b32 %0, %2, %1" : "=v"(x) : "v"(off), "n"(kXor));
+  if constexpr (kAdd != 0) asm volatile("v_add_u32 %0, %2, %1" : "=v"(x) : "v"(x), "n"(kAdd));
+  return x;
+}
+// load_lds_b128 with an instruction offset, which the hardware adds to both the
+// memory and the LDS address.
+template <int kOffset>
+__device__ __forceinline__ void load_lds_b128_at(const void *base, std::uint32_t voff, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%3"
+               :
+               : "s"(lds), "v"(voff), "s"(base), "n"(kOffset)
+               : "memory");
+}
+
+// The O^T accumulators (2 column blocks x 8 dim blocks x 16 registers) fill the
+// 256 accumulation registers, and are addressed by number from asm: block
+// `kAcc` (8 b + nb) is a[16 kAcc : 16 kAcc + 15].  Left to the register
+// allocator, values of this size were copied and spilled around every tile.
+// acc_fence clobbers the whole file around every tile, so the compiler keeps
+// nothing of its own there (the statements in between carry no clobber list,
+// which took minutes to compile); the build checks that no instruction outside
+// asm uses an accumulation register (raftinfer_amd/asm_check.py).
+#define RAFT_AGPR10(n) \
+  "a" #n "0", "a" #n "1", "a" #n "2", "a" #n "3", "a" #n "4", "a" #n "5", "a" #n "6", "a" #n "7", "a" #n "8", "a" #n "9"
+#define RAFT_ALL_AGPRS \
+  "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", \
+      RAFT_AGPR10(1), RAFT_AGPR10(2), RAFT_AGPR10(3), RAFT_AGPR10(4), \
+      RAFT_AGPR10(5), RAFT_AGPR10(6), RAFT_AGPR10(7), RAFT_AGPR10(8), \
+      RAFT_AGPR10(9), RAFT_AGPR10(10), RAFT_AGPR10(11), RAFT_AGPR10(12), \
+      RAFT_AGPR10(13), RAFT_AGPR10(14), RAFT_AGPR10(15), RAFT_AGPR10(16), \
+      RAFT_AGPR10(17), RAFT_AGPR10(18), RAFT_AGPR10(19), RAFT_AGPR10(20), \
+      RAFT_AGPR10(21), RAFT_AGPR10(22), RAFT_AGPR10(23), RAFT_AGPR10(24), \
+      "a250", "a251", "a252", "a253", "a254", "a255"
+
+__device__ __forceinline__ void acc_fence() { asm volatile("" : : : RAFT_ALL_AGPRS); }
+template <int kAcc> __device__ __forceinline__ void acc_mfma(bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 a[%0:%1], %2, %3, a[%0:%1]"
+               :
+               : "n"(16 * kAcc), "n"(16 * kAcc + 15), "v"(a), "v"(b));
+}
+// s = a b and s += a b with s in vector registers.  A statement writes no
+// result for another 19 wait states: new_max reads S(t + 4) only after PV(t),
+// and after the first tile's chain the kernel drains.
+__device__ __forceinline__ void s_mfma_zero(floatx16 &s, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(s) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void s_mfma(floatx16 &s, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(s) : "v"(a), "v"(b));
+}
+template <int kReg> __device__ __forceinline__ void acc_set(float x) {
+  asm volatile("v_accvgpr_write_b32 a[%0], %1" : : "n"(kReg), "v"(x));
+}
+template <int kReg> __device__ __forceinline__ float acc_get() {
+  float x;
+  asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(x) : "n"(kReg));
+  return x;
+}
+// max(a, b, c).  As asm: on results of the asm MFMAs fmaxf adds a canonicalising
+// instruction per operand.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  float x;
+  asm volatile("v_max3_f32 %0, %1, %2, %3" : "=v"(x) : "v"(a), "v"(b), "v"(c));
+  return x;
+}
+// The wait states between the last s_mfma of a chain and the first use of s.
+template <int NB> __device__ __forceinline__ void s_drain(floatx16 (&s)[NB]) {
+  if constexpr (NB == 2)
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(s[0]), "+v"(s[1]));
+  else
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(s[0]));
+}
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>)
+template <int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
+  [&]<int... I>(std::integer_sequence<int, I...>) __attribute__((always_inline)) { (f(std::integral_constant<int, I>{}), ...); }
+  (std::make_integer_sequence<int, N>{});
+}
+
+// NB column blocks of 32 per wave, KS key groups (see the head of the file).
+template <int NB, int KS> struct Plan {
+  static constexpr int kShare = kWaves / KS;            // waves that share a key group's tiles
+  static constexpr int kTok = 8 * NB * kShare;          // query tokens per workgroup
+  static constexpr int kRows = 4 * kTok;                // columns, one staged row each
+  static constexpr unsigned kSlot = 8192u * kShare;     // ring slot: 16 / 32 rows of 512 bytes
+  static constexpr unsigned kArea = 5 * kSlot;          // a key group's part of LDS
+  static constexpr int kGroupRows = kRows / KS;         // staged rows in each group's area
+  static constexpr unsigned kRowsAt = kShare == 1 ? 4 * kSlot : 3 * kSlot;
+  static constexpr int kParts = 8 / KS;                 // dims blocks that a wave finishes
+};
+
+template <int NB, int KS, bool HeadMajor, bool FromInput, bool NormQ>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_wide_kernel(
+    const bf16_bits *__restrict__ query, const bf16_bits *key_in, const bf16_bits *value_in,
+    const bf16_bits *gate, bf16_bits *__restrict__ output, bf16_bits *__restrict__ cache,
+    std::size_t tokens, std::size_t max_ctx, std::size_t past, PrefillNormRope nq) {
+  static_assert(!(NormQ && FromInput), "the fused producer path reads K/V from the cache");
+  using P = Plan<NB, KS>;
+  constexpr int kTok = P::kTok, kShare = P::kShare;
+  constexpr unsigned kSlot = P::kSlot;
+  __shared__ __attribute__((aligned(16384))) unsigned char sh[KS * P::kArea];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int col = lane & 31;  // MFMA column of a block: head_in_group * 8 + token
+  const int half = lane >> 5; // k-half of the MFMA operands
+  const std::size_t n_qtiles = ceil_div_u(tokens, kTok);
+  const unsigned xcd = blockIdx.x & 7u;
+  const std::size_t slot_index = 2 * (blockIdx.x >> 3) + (xcd & 1u);
+  if (slot_index >= n_qtiles) return; // padding of an odd tile count
+  const std::size_t qtile = n_qtiles - 1 - slot_index;
+  const std::size_t kv_head = xcd >> 1;
+  const std::size_t t0 = qtile * kTok;
+  const std::size_t q_rows = tokens - t0 < kTok ? tokens - t0 : kTok;
+  const std::size_t key_end = past + t0 + q_rows;
+  const std::size_t n_tiles = (key_end + kKTile - 1) / kKTile;
+  const std::size_t plane = max_ctx * kKvHeads * kHeadDim;
+  const float scale = kLog2e / 16.0f;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave % KS, cg = wave / KS; // key group, column group
+  // Token slot of staged row r = 32 blk + c, clamped to the tile's tokens, and
+  // the element offset of its row in the query / gate / output layout [T][16][256].
+  auto slot_row = [&](int r) __attribute__((always_inline)) {
+    const std::size_t tt = 8 * (r >> 5) + (r & 7);
+    return tt < q_rows ? tt : q_rows - 1;
+  };
+  auto io_row = [&](int r) __attribute__((always_inline)) {
+    return ((t0 + slot_row(r)) * kQueryHeads + kv_head * kGroup + ((r & 31) >> 3)) * kHeadDim;
+  };
+  constexpr std::size_t q_row_elems = NormQ ? 2 * kHeadDim : kHeadDim;
+  const bf16_bits *gate_src = NormQ ? query + kHeadDim : gate;
+  const unsigned lds0 = lds_address(sh);
+  const unsigned ring = lds0 + kg * P::kArea;
+  // LDS address of a staged row (Q, gate, output): 16-byte chunk k at k ^ swz(r).
+  auto row_at = [&](int r) __attribute__((always_inline)) {
+    return lds0 + (r / P::kGroupRows) * P::kArea + P::kRowsAt + (r % P::kGroupRows) * 512u;
+  };
+
+  // The lane index again: what is derived from it is not computed before the tile
+  // loop and kept (or spilled) over it.
+  auto late_lane = [&]() __attribute__((always_inline)) {
+    int l = threadIdx.x & 63;
+    asm volatile("" : "+v"(l));
+    return l;
+  };
+  // ---- staging: ring items of 8 loads (1 KiB) per wave.
+  //   K, own tiles: one dims half of the 32-key tile, 4 half-rows a load (rows
+  //     4i + lane / 16), 16-byte chunk c (0..15) at c ^ f, f = 4 (row % 4) + row / 4 % 4;
+  //   K, shared tiles: 16 rows, two whole rows a load (2i + lane / 32), chunk c
+  //     (0..31) at c ^ f, f = row / 2 % 8 + 8 (row % 2);
+  //   V: 16 rows likewise, f = 4 (row / 2 % 2) + 8 (row % 2).
+  // The 16 rows of a ds_read_b128 pass over K then share no bank, nor do the 4
+  // rows x 64 bytes of a ds_read_b64_tr_b16 pass over V, whose rows 8 apart have
+  // the same f.  A load's offset is the lane's, an exclusive-or and an addition.
+  constexpr std::uint32_t row_bytes = HeadMajor && !FromInput ? kHeadDim * 2 : kKvHeads * kHeadDim * 2;
+  const bf16_bits *k_src = FromInput ? key_in + kv_head * kHeadDim
+                                     : cache + cache_row(HeadMajor, 0, kv_head, max_ctx);
+  const bf16_bits *v_src = FromInput ? value_in + kv_head * kHeadDim : k_src + plane;
+  constexpr int k_rows = kShare == 1 ? 4 : 2; // rows per K load
+  const int hrow = kShare == 1 ? lane >> 4 : half;
+  const std::uint32_t v_off = half * row_bytes + 16u * (col ^ (8 * half));
+  const std::uint32_t k_off = kShare == 1 ? hrow * row_bytes + 16u * ((lane & 15) ^ (4 * hrow)) : v_off;
+  auto load_k = [&](const unsigned char *base, unsigned to, auto ic) __attribute__((always_inline)) {
+    constexpr int i = ic, x = kShare == 1 ? i & 3 : i;
+    load_lds_b128_at<1024 * (i & 3)>(base + 4096 * (i >> 2), load_offset<16u * x, i *(k_rows * row_bytes - 1024)>(k_off),
+                                     to + 4096u * (i >> 2));
+  };
+  auto load_v = [&](const unsigned char *base, unsigned to, auto ic) __attribute__((always_inline)) {
+    constexpr int i = ic;
+    load_lds_b128_at<1024 * (i & 3)>(base + 4096 * (i >> 2), load_offset<64u * (i & 1), i *(2 * row_bytes - 1024)>(v_off),
+                                     to + 4096u * (i >> 2));
+  };
+  auto base_of = [&](const bf16_bits *src, std::size_t row) __attribute__((always_inline)) {
+    return reinterpret_cast<const unsigned char *>(src) + row * row_bytes;
+  };
+  // The same for items that may reach past key_end: those rows re-read the last
+  // one (their scores are masked).  k0: first row; for K of own tiles `half_tile`
+  // is the dims half.
+  auto load_clamped = [&](const bf16_bits *src, auto is_v, std::size_t k0, int half_tile, unsigned to, auto ic)
+      __attribute__((always_inline)) {
+    constexpr int i = ic;
+    constexpr bool dims_half = kShare == 1 && !is_v;
+    const std::size_t first = k0 < key_end ? k0 : key_end - 1;
+    const std::uint32_t last = static_cast<std::uint32_t>(key_end - 1 - first < 31 ? key_end - 1 - first : 31);
+    const int l = late_lane();
+    const std::uint32_t r = dims_half ? 4 * i + (l >> 4) : 2 * i + (l >> 5);
+    const std::uint32_t chunk = dims_half ? (l & 15) ^ (4 * (l >> 4)) ^ (i & 3)
+                                          : (l & 31) ^ (8 * (l >> 5)) ^ (is_v ? 4 * (i & 1) : i);
+    // (no instruction offset here: less 1024 i, the offset of a clamped row could
+    // be negative, and it is unsigned)
+    load_lds_b128_at<0>(base_of(src, first) + (dims_half ? 256 * half_tile : 0), (r < last ? r : last) * row_bytes + 16u * chunk,
+                        to + 1024u * i);
+  };
+  // Tile of this wave's key group, counted from its first, and the first row of
+  // its share `sub` of it.
+  auto tile_row = [&](std::size_t n, int sub) __attribute__((always_inline)) {
+    return (n * KS + kg) * kKTile + 16 * sub;
+  };
+  constexpr std::false_type kIsK{};
+  constexpr std::true_type kIsV{};
+  auto load_item = [&](const bf16_bits *src, auto is_v, std::size_t k0, int half_tile, unsigned to)
+      __attribute__((always_inline)) {
+    static_for<8>([&](auto i) __attribute__((always_inline)) { load_clamped(src, is_v, k0, half_tile, to, i); });
+  };
+  // This wave's kRows / 4 staged rows from a [T][16][row elems] source, two per load.
+  auto issue_rows = [&](const bf16_bits *src, int lane) __attribute__((always_inline)) {
+    constexpr int n = P::kRows / kWaves;
+    const unsigned to = row_at(n * wave);
+#pragma unroll
+    for (int i = 0; i < n / 2; ++i) {
+      const int r = n * wave + 2 * i + (lane >> 5);
+      const std::uint32_t voff =
+          static_cast<std::uint32_t>(slot_row(r) * kQueryHeads + ((r & 31) >> 3)) * (q_row_elems * 2) +
+          16u * ((lane & 31) ^ swz(r));
+      load_lds_b128(src + (t0 * kQueryHeads + kv_head * kGroup) * q_row_elems, voff, to + 1024u * i);
+    }
+  };
+  // Tiles of this key group; with shared tiles every wave runs the same number
+  // (the barriers), the tiles past n_tiles fully masked.
+  const std::size_t m = kShare > 1 ? ceil_div_u(n_tiles, KS)
+                                   : (n_tiles > static_cast<std::size_t>(kg) ? ceil_div_u(n_tiles - kg, KS) : 0);
+  // Ring items of 8 loads per wave each (i = tile):
+  //   own tiles (half tiles h):     K0 K1(0) K0 K1(1) V0 V1(0) K0 K1(2) V0 V1(1) ...
+  //   shared tiles (whole tiles):   K(0) K(1) V(0) K(2) V(1) K(3) V(2) ...
+  // Item n uses slot n % 5.  While item n is read, item n + 4 is loaded into the
+  // slot of n - 1 (own tiles), or item n + 3 into the slot of n - 2, which every
+  // wave has left when it passes the barrier in front of item n (shared tiles).
+  issue_rows(query, lane);
+  const int my = kShare > 1 ? cg : 0; // this wave's share of an item
+  const unsigned part = 8192u * my;
+  auto issue_start = [&](int from, int to) __attribute__((always_inline)) {
+    if constexpr (kShare == 1) {
+      for (int n = from; n < to; ++n)
+        if (static_cast<std::size_t>(n >> 1) < m) load_item(k_src, kIsK, tile_row(n >> 1, 0), n & 1, ring + n * kSlot);
+    } else {
+      for (int n = from; n < to; ++n)
+        if (n == 0) load_item(k_src, kIsK, tile_row(0, my), 0, ring + part);
+        else if (n == 1 && m > 1) load_item(k_src, kIsK, tile_row(1, my), 0, ring + kSlot + part);
+        else if (n == 2) load_item(v_src, kIsV, tile_row(0, my), 0, ring + 2 * kSlot + part);
+    }
+  };
+  constexpr int kFirstItems = kShare == 1 ? 2 : 1; // before the norm, 2 / 1 items (K(0))
+  constexpr int kStartItems = kShare == 1 ? 4 : 3;
+  if constexpr (NormQ) {
+    // The norm weight (512 B bf16 or 1 KiB f32) into the second-last group's
+    // slot 2, the rotation tables of the tile's (up to kTok) positions into the
+    // last group's slots 2, 3 (own tiles) or 1, 2; the items of those slots go
+    // out once they have been used.
+    const unsigned w_at = lds0 + (KS - 2) * P::kArea + 2 * kSlot;
+    const unsigned rot_at = lds0 + (KS - 1) * P::kArea + (kShare == 1 ? 2 : 1) * kSlot;
+    if (wave == 0) {
+      const std::uint32_t bytes = nq.weight_f32 ? 1024u : 512u;
+      const std::uint32_t off = 16u * lane < bytes ? 16u * lane : bytes - 16u;
+      load_lds_b128(nq.weight, off, w_at);
+    }
+    issue_start(0, kFirstItems);
+    auto rot = reinterpret_cast<float(*)[kHeadDim]>(lds_ptr<float>(rot_at));
+    for (int i = tid; i < kTok * nq.pairs; i += kThreads) {
+      const int s = i / nq.pairs, pp = i - s * nq.pairs;
+      const std::size_t tt = static_cast<std::size_t>(s) < q_rows ? s : q_rows - 1;
+      float cs, sn;
+      rope_cos_sin(pp, past + t0 + tt, nq.ratio, cs, sn);
+      rot[s][pp] = cs;
+      rot[s][nq.pairs + pp] = sn;
+    }
+    if (m != 0) wait_vm<8 * kFirstItems>(); else wait_vm<0>();
+    __syncthreads();
+    const float *weight = lds_ptr<float>(w_at);
+    constexpr int n = P::kRows / kWaves;
+#pragma unroll
+    for (int g8 = 0; g8 < n / 8; ++g8) { // eight rows (one head, the 8 token slots of a block) at a time
+      const int row0 = n * wave + 8 * g8;
+      const float(*rows)[kHeadDim] = rot + 8 * (row0 >> 5);
+      bf16_bits *staged = lds_ptr<bf16_bits>(row_at(row0));
+      if (nq.pairs % 32 == 0)
+        norm_rope_rows_sliced(staged, lane >> 3, lane & 7, weight, nq.weight_f32, nq.pairs, rows[lane >> 3],
+                              nq.epsilon);
+      else
+        norm_rope_rows_lanewise(staged, 0, lane, weight, nq.weight_f32, nq.pairs, rows, nq.epsilon);
+    }
+    __syncthreads(); // every row is normalised, the tables have been read
+    issue_start(kFirstItems, kStartItems);
+  } else {
+    issue_start(0, kStartItems);
+  }
+  acc_fence();
+  static_for<128 * NB>([](auto r) __attribute__((always_inline)) { acc_set<r>(0.f); });
+  acc_fence();
+  float m_run[NB], l_run[NB]; // reference max (exp2 domain) and this lane's sum, of column `col`
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    m_run[b] = -INFINITY;
+    l_run[b] = 0.f;
+  }
+  if constexpr (!NormQ) {
+    // this wave's Q rows have landed, then every other wave's
+    if constexpr (kShare == 1) {
+      if (m > 1) wait_vm<32>(); else if (m != 0) wait_vm<16>(); else wait_vm<0>();
+    } else {
+      if (m > 1) wait_vm<24>(); else wait_vm<16>();
+    }
+    __syncthreads();
+  }
+  // Q^T operands stay in registers: block b, k-step kk holds chunk 2 kk + half
+  // of the staged row of its column.
+  bf16x8 qa[NB][16];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const unsigned row = row_at(32 * (NB * cg + b) + col);
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) qa[b][kk] = lds_read_b128(row + 16u * ((2 * kk + half) ^ swz(col)));
+  }
+  wait_lgkm0();
+  __syncthreads(); // the staged rows' slots are free
+
+  // Slot addresses of ring items n - 1, n, n + 1, n + 2, n + 3 (n = the next to
+  // be read); the slot of n - 2 is that of n + 3.
+  unsigned p0 = ring + 4 * kSlot, p1 = ring, p2 = ring + kSlot, p3 = ring + 2 * kSlot, p4 = ring + 3 * kSlot;
+  auto advance = [&](int items) __attribute__((always_inline)) {
+    for (int i = 0; i < items; ++i) {
+      const unsigned x = p0;
+      p0 = p1; p1 = p2; p2 = p3; p3 = p4; p4 = x;
+    }
+  };
+  // K operand of k-step kk: chunk 2 kk + half of row col.  V^T operand
+  // (transposed read) of dims block nb and key step kb: rows 16 kb + 4 half +
+  // r / 4 and 8 below, dims 32 nb + 16 (g & 1) + 4 (r & 3).
+  const unsigned k_lane = kShare == 1 ? col * 256u + 16u * (half ^ (4 * (col & 3) + ((col >> 2) & 3)))
+                                      : col * 512u + 16u * (half ^ (((col >> 1) & 7) + 8 * (col & 1)));
+  const int vg = (lane >> 4) & 1, vr = lane & 15, vrow = 4 * half + (vr >> 2);
+  const unsigned v_lane = vrow * 512u + 16u * ((2 * vg + ((vr & 3) >> 1)) ^ (4 * ((vrow >> 1) & 1) + 8 * (vrow & 1))) +
+                          8u * (vr & 1);
+  bf16x8 op[4];       // operands of the next four MFMA groups, across phases
+  unsigned at = 0;    // lane address of the tile part being read
+  unsigned at_x = 0;  // ... of the exclusive-or group being read
+  // Order within a phase, s = 0..15: with own tiles k-step s (the dims halves
+  // one after the other), with shared tiles k-steps s / 2 and s / 2 + 8 in turn;
+  // for V, key step s / 8 and dims blocks s / 2 % 4 and s / 2 % 4 + 4 in turn.
+  // Such pairs share their exclusive-or.
+  auto k_operand = [&](auto sc) __attribute__((always_inline)) {
+    constexpr int s = sc;
+    if constexpr (kShare == 1) return lds_read_b128(at ^ (32u * (s & 7)));
+    if constexpr (s % 2 == 0) at_x = at ^ (32u * (s >> 1));
+    return lds_read_b128(at_x + 256u * (s & 1));
+  };
+  auto v_operand = [&](auto sc) __attribute__((always_inline)) {
+    constexpr int s = sc;
+    constexpr unsigned off = 256u * (s & 1) + (kShare > 1 ? 8192u * (s >> 3) : 0u);
+    if constexpr (s % 2 == 0) at_x = at ^ (64u * ((s >> 1) & 3));
+    const u32x2 lo = lds_read_tr16(at_x + off), hi = lds_read_tr16(at_x + off + 4096u);
+    return __builtin_bit_cast(bf16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+  };
+
+  floatx16 s0[NB], s1[NB];
+  std::uint32_t pk[NB][8]; // P^T, bf16 pairs in accumulator order
+  float m_ref[NB], mx[NB]; // mx: max of the next S over this lane's keys
+
+  // Pair u of the probabilities (blocks in turn): registers 2i, 2i+1 of an S.
+  // The sum takes the same bf16 probabilities as the PV product.  The empty asm
+  // keeps the pair where it is written, among the MFMAs.
+  auto soft_pair = [&](const floatx16(&s)[NB], auto uc) __attribute__((always_inline)) {
+    constexpr int b = uc % NB, i = uc / NB;
+    const float x0 = fexp2(fmaf(s[b][2 * i], scale, -m_ref[b]));
+    const float x1 = fexp2(fmaf(s[b][2 * i + 1], scale, -m_ref[b]));
+    pk[b][i] = pack_bf16x2(x0, x1);
+    l_run[b] = dot2_bf16(pk[b][i], 0x3F803F80u, l_run[b]);
+    asm volatile("" : "+v"(pk[b][i]), "+v"(l_run[b]));
+  };
+  // Pairs [A, B) spread over the steps of a part of `steps` steps.
+  auto soft_step = [&](const floatx16(&s)[NB], auto sc, auto from, auto count, auto steps) __attribute__((always_inline)) {
+    constexpr int u0 = sc * count / steps, u1 = (sc + 1) * count / steps;
+    static_for<u1 - u0>([&](auto k) __attribute__((always_inline)) {
+      soft_pair(s, std::integral_constant<int, from + u0 + k>{});
+    });
+  };
+  constexpr std::integral_constant<int, 0> c0{};
+  constexpr std::integral_constant<int, 6 * NB> kQkPairs{}; // of 8 NB; all of key step 0 among them
+  constexpr std::integral_constant<int, 2 * NB> kPvPairs{};
+  constexpr std::integral_constant<int, 16> c16{};
+  constexpr std::integral_constant<int, 8> c8{};
+  auto lane_max = [&](const floatx16(&s)[NB]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      mx[b] = max3(s[b][0], s[b][1], s[b][2]);
+#pragma unroll
+      for (int i = 3; i < 15; i += 2) mx[b] = max3(mx[b], s[b][i], s[b][i + 1]);
+      mx[b] = max3(mx[b], s[b][15], s[b][15]);
+    }
+  };
+  // The new reference max from mx, and the (rare) rescale of the accumulators:
+  // it moves only when a column max grows by more than 2^8.
+  auto new_max = [&](bool first) __attribute__((always_inline)) {
+    float mm[NB];
+    bool grow[NB], any_grow = false;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      mm[b] = max_xor32(mx[b]) * scale;
+      grow[b] = mm[b] > m_run[b] + kLazyRescale;
+      any_grow |= grow[b];
+    }
+    if (first) { // nothing is accumulated yet
+#pragma unroll
+      for (int b = 0; b < NB; ++b) m_run[b] = grow[b] ? mm[b] : m_run[b];
+    } else if (__builtin_amdgcn_ballot_w64(any_grow) != 0) {
+      mfma_drain();
+      static_for<NB>([&](auto b) __attribute__((always_inline)) {
+        const float sc = grow[b] ? fexp2(m_run[b] - mm[b]) : 1.0f;
+        l_run[b] *= sc;
+        m_run[b] = grow[b] ? mm[b] : m_run[b];
+        static_for<128>([&](auto r) __attribute__((always_inline)) { acc_set<128 * b + r>(acc_get<128 * b + r>() * sc); });
+      });
+    }
+    // a column whose keys so far are all masked keeps m = -inf
+#pragma unroll
+    for (int b = 0; b < NB; ++b) m_ref[b] = m_run[b] == -INFINITY ? 0.f : m_run[b];
+  };
+  // Keys past each column's position score -inf (register i: key 8 (i / 4) +
+  // 4 half + i % 4 of the tile at row k0).
+  auto mask = [&](floatx16(&s)[NB], std::size_t k0) __attribute__((always_inline)) {
+    const int le = late_lane();
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const std::ptrdiff_t rel = static_cast<std::ptrdiff_t>(past + t0 + slot_row(32 * (NB * cg + b) + (le & 31))) -
+                                 static_cast<std::ptrdiff_t>(k0) - 4 * (le >> 5);
+      const int lim = rel < -1 ? -1 : (rel > kKTile ? kKTile : static_cast<int>(rel));
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[b][i] = (i >> 2) * 8 + (i & 3) > lim ? -INFINITY : s[b][i];
+    }
+    lane_max(s);
+  };
+  auto none = [](auto) __attribute__((always_inline)) {};
+  // Waits until the wave's share of the next ring item has landed, with n of its
+  // later loads outstanding, and with shared tiles until every wave's has.
+  auto ready = [&](auto n) __attribute__((always_inline)) {
+    wait_vm<n>();
+    if constexpr (kShare > 1) __builtin_amdgcn_s_barrier();
+  };
+  // out = K Q^T of the tile at `at`, on the matrix unit, while (soft) the vector
+  // unit turns s into probabilities.  load(step) issues the wave's loads of this
+  // phase, second_ready / next_ready wait for the second half tile and for V.
+  auto qk = [&](auto soft, const floatx16(&s)[NB], floatx16(&out)[NB], auto load, auto second_ready, auto next_ready,
+                unsigned k_second, unsigned v_slot)
+      __attribute__((always_inline)) {
+    static_for<16>([&](auto st) __attribute__((always_inline)) {
+      constexpr int q = st & 3, kk = kShare == 1 ? +st : (st >> 1) + 8 * (st & 1);
+      if constexpr (st == 0) s_mfma_zero(out[0], op[q], qa[0][kk]); else s_mfma(out[0], op[q], qa[0][kk]);
+      if constexpr (soft) soft_step(s, st, c0, kQkPairs, c16);
+      if constexpr (NB == 2) {
+        if constexpr (st == 0) s_mfma_zero(out[1], op[q], qa[1][kk]); else s_mfma(out[1], op[q], qa[1][kk]);
+      }
+      if constexpr (kShare == 1 && st == 4) {
+        second_ready();
+        at = k_second + k_lane;
+      }
+      if constexpr (soft && st == 12) {
+        next_ready();
+        at = v_slot + v_lane;
+      }
+      if constexpr (st < 12) op[q] = k_operand(std::integral_constant<int, st + 4>{});
+      else if constexpr (soft) op[q] = v_operand(std::integral_constant<int, st - 12>{});
+      load(st);
+      if constexpr (st % 2 == 1) acc_fence();
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  // O += V^T P^T, the remaining probabilities of s formed on the way; with kMax
+  // the max of `next` over this lane's keys is taken and the next K tile begun.
+  auto pv = [&](auto kMax, const floatx16(&s)[NB], const floatx16(&next)[NB], auto load, auto second_ready,
+                auto next_ready, unsigned v_second, unsigned k_a) __attribute__((always_inline)) {
+    acc_fence();
+    auto p_operand = [&](int b, int kb) __attribute__((always_inline)) {
+      return __builtin_bit_cast(bf16x8, u32x4{pk[b][4 * kb], pk[b][4 * kb + 1], pk[b][4 * kb + 2], pk[b][4 * kb + 3]});
+    };
+    static_for<16>([&](auto st) __attribute__((always_inline)) {
+      constexpr int q = st & 3, kb = st >> 3, nb = ((st >> 1) & 3) + 4 * (st & 1);
+      acc_mfma<nb>(op[q], p_operand(0, kb));
+      if constexpr (st < 8) soft_step(s, st, kQkPairs, kPvPairs, c8);
+      if constexpr (NB == 2) acc_mfma<8 + nb>(op[q], p_operand(1, kb));
+      if constexpr (st == 4 && kShare == 1) {
+        second_ready();
+        at = v_second + v_lane;
+      }
+      if constexpr (kMax && st == 12) {
+        next_ready();
+        at = k_a + k_lane;
+      }
+      if constexpr (st < 12) op[q] = v_operand(std::integral_constant<int, st + 4>{});
+      else if constexpr (kMax) op[q] = k_operand(std::integral_constant<int, st - 12>{});
+      if constexpr (kMax && st >= 8) { // two values of each block per step
+        constexpr int i = 2 * (st - 8);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) mx[b] = max3(st == 8 ? next[b][0] : mx[b], next[b][i], next[b][i + 1]);
+      }
+      load(st);
+      if constexpr (st % 4 == 3) acc_fence();
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+
+  // Step n: tile n (its S in s, mx its max) -> O, with S(n + 1) formed on the
+  // way.  kSteady: every item loaded in the step exists and is whole.  The two S
+  // buffers alternate by name: a copy placed right behind the MFMA that writes
+  // it would read it too early.
+  std::size_t n = 0;
+  const std::size_t full = key_end / kKTile; // whole tiles, then those of the group
+  const std::size_t whole = full > static_cast<std::size_t>(kg) ? ceil_div_u(full - kg, KS) : 0;
+  auto step = [&](auto kSteady, floatx16(&s)[NB], floatx16(&next)[NB]) __attribute__((always_inline)) {
+    if constexpr (!kSteady)
+      if (tile_row(n, 0) + kKTile - 1 > past + t0) mask(s, tile_row(n, 0));
+    new_max(n == 0);
+    if constexpr (kShare == 1) {
+      // QK reads K(n+1) (items n', n'+1) and loads K(n+2), PV reads V(n) and loads V(n+1).
+      const bool more = kSteady || n + 2 < m;
+      auto wait = [&]() __attribute__((always_inline)) { if (more) wait_vm<20>(); else wait_vm<4>(); };
+      const unsigned char *kb0 = base_of(k_src, tile_row(n + 2, 0)), *vb0 = base_of(v_src, tile_row(n + 1, 0));
+      qk(std::true_type{}, s, next,
+         [&](auto st) __attribute__((always_inline)) {
+           constexpr std::integral_constant<int, st & 7> i{};
+           const unsigned to = st < 8 ? p0 : p1;
+           if constexpr (kSteady) load_k(st < 8 ? kb0 : kb0 + 256, to, i);
+           else if (more) load_clamped(k_src, kIsK, tile_row(n + 2, 0), st >> 3, to, i);
+         },
+         wait, wait, p2, p3);
+      pv(std::true_type{}, s, next,
+         [&](auto st) __attribute__((always_inline)) {
+           constexpr std::integral_constant<int, st & 7> i{};
+           const unsigned to = st < 8 ? p2 : p3; // V0(n) has been read after half the phase
+           if constexpr (kSteady) load_v(st < 8 ? vb0 : vb0 + 16 * row_bytes, to, i);
+           else load_clamped(v_src, kIsV, tile_row(n + 1, st >> 3), 0, to, i);
+         },
+         wait, wait, p4, p0);
+      advance(4);
+    } else {
+      // QK reads K(n+1) and loads V(n+1), PV reads V(n) and loads K(n+3).
+      const bool more2 = kSteady || n + 2 < m, more3 = kSteady || n + 3 < m;
+      const unsigned char *vb0 = base_of(v_src, tile_row(n + 1, my)), *kb0 = base_of(k_src, tile_row(n + 3, my));
+      qk(std::true_type{}, s, next,
+         [&](auto st) __attribute__((always_inline)) {
+           if constexpr (st % 2 == 0) {
+             constexpr std::integral_constant<int, st / 2> i{};
+             const unsigned to = p4 + part; // item n' + 3
+             if constexpr (kSteady) load_v(vb0, to, i);
+             else load_clamped(v_src, kIsV, tile_row(n + 1, my), 0, to, i);
+           }
+         },
+         [] {}, [&]() __attribute__((always_inline)) { if (more2) ready(std::integral_constant<int, 14>{}); else ready(std::integral_constant<int, 6>{}); },
+         0, p2);
+      pv(std::true_type{}, s, next,
+         [&](auto st) __attribute__((always_inline)) {
+           if constexpr (st % 2 == 0) {
+             constexpr std::integral_constant<int, st / 2> i{};
+             const unsigned to = p0 + part; // item n' + 4, the slot of n' - 1
+             if constexpr (kSteady) load_k(kb0, to, i);
+             else if (more3) load_clamped(k_src, kIsK, tile_row(n + 3, my), 0, to, i);
+           }
+         },
+         [] {},
+         [&]() __attribute__((always_inline)) { if (more3) ready(std::integral_constant<int, 14>{}); else ready(std::integral_constant<int, 0>{}); },
+         0, p3);
+      advance(2);
+    }
+    ++n;
+  };
+  if (m != 0) {
+    // S of the first tile: items 0, 1 (own) or 0 (shared) are read, V(0) or K(2) loaded.
+    if constexpr (kShare == 1) {
+      if (m > 1) wait_vm<24>(); else wait_vm<8>(); // K(0), first half
+      at = p1 + k_lane;
+      static_for<4>([&](auto i) __attribute__((always_inline)) { op[i] = k_operand(i); });
+      qk(std::false_type{}, s0, s0,
+         [&](auto st) __attribute__((always_inline)) {
+           load_clamped(v_src, kIsV, tile_row(0, st >> 3), 0, st < 8 ? p0 : p1,
+                        std::integral_constant<int, st & 7>{});
+         },
+         [&]() __attribute__((always_inline)) { if (m > 1) wait_vm<20>(); else wait_vm<4>(); }, [] {}, p2, 0);
+      advance(2);
+    } else {
+      if (m > 1) wait_vm<16>(); else wait_vm<8>();
+      __builtin_amdgcn_s_barrier();
+      at = p1 + k_lane;
+      static_for<4>([&](auto i) __attribute__((always_inline)) { op[i] = k_operand(i); });
+      qk(std::false_type{}, s0, s0,
+         [&](auto st) __attribute__((always_inline)) {
+           if constexpr (st % 2 == 0)
+             if (m > 2) load_clamped(k_src, kIsK, tile_row(2, my), 0, p4 + part, std::integral_constant<int, st / 2>{});
+         },
+         [] {}, [] {}, 0, 0);
+      advance(1);
+    }
+    s_drain(s0);
+    lane_max(s0);
+    if (m > 1) { // K(1)
+      if constexpr (kShare == 1)
+        wait_vm<24>(); // first half
+      else if (m > 2)
+        ready(std::integral_constant<int, 16>{});
+      else
+        ready(std::integral_constant<int, 8>{});
+      at = p1 + k_lane;
+      static_for<4>([&](auto i) __attribute__((always_inline)) { op[i] = k_operand(i); });
+    }
+    constexpr std::size_t kReach = kShare == 1 ? 2 : 3; // the furthest tile that a step loads
+    while (n + kReach + 1 < whole) {
+      step(std::true_type{}, s0, s1);
+      step(std::true_type{}, s1, s0);
+    }
+    while (n + 1 < m) {
+      step(std::false_type{}, s0, s1);
+      if (n + 1 >= m) {
+        s_drain(s1);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) s0[b] = s1[b];
+        break;
+      }
+      step(std::false_type{}, s1, s0);
+    }
+    if (tile_row(n, 0) + kKTile - 1 > past + t0) mask(s0, tile_row(n, 0));
+    new_max(n == 0);
+    static_for<kQkPairs>([&](auto u) __attribute__((always_inline)) { soft_pair(s0, u); });
+    if constexpr (kShare == 1) {
+      wait_vm<8>(); // V(last), first half
+      at = p3 + v_lane;
+    } else {
+      ready(std::integral_constant<int, 0>{});
+      at = p2 + v_lane;
+    }
+    static_for<4>([&](auto i) __attribute__((always_inline)) { op[i] = v_operand(i); });
+    pv(std::false_type{}, s0, s0, none, [] { wait_vm<0>(); }, [] {}, p4, 0);
+    mfma_drain();
+    wait_lgkm0();
+  }
+  // ---- epilogue.  The gate rows take the staged rows' place, and the partials
+  // are merged one column block at a time: wave (kg, cg) finishes dims 256 / KS
+  // kg .. of the columns that it shares with the other waves of column group cg.
+  if constexpr (kShare > 1) __syncthreads(); // every wave has left the ring
+  const int lane_e = late_lane(), col_e = lane_e & 31, half_e = lane_e >> 5;
+  issue_rows(gate_src, lane_e);
+  constexpr int kApp = FromInput ? kTok / 4 : 1; // this workgroup's cache rows: 2 planes x kTok tokens x 32 pieces
+  [[maybe_unused]] u32x4 app[kApp];
+  auto app_at = [&](int j, int &pl, int &tok, int &piece) __attribute__((always_inline)) {
+    const int idx = kWave * wave + lane_e + kThreads * j;
+    pl = idx / (kTok * 32);
+    tok = (idx >> 5) % kTok;
+    piece = idx & 31;
+  };
+  if constexpr (FromInput) {
+#pragma unroll
+    for (int j = 0; j < kApp; ++j) {
+      int pl, tok, piece;
+      app_at(j, pl, tok, piece);
+      const std::size_t tt = static_cast<std::size_t>(tok) < q_rows ? tok : q_rows - 1;
+      app[j] = *reinterpret_cast<const u32x4 *>((pl ? value_in : key_in) +
+                                                ((t0 + tt) * kKvHeads + kv_head) * kHeadDim + 8 * piece);
+    }
+  }
+  // Partials of wave (g, cg) for the finisher of part q (q != g): [dims block of
+  // the part][register quad][lane] float4; its (max, sum) of each block, [2 NB][lane].
+  constexpr unsigned kPartBytes = P::kParts * 4 * kWave * sizeof(float4);
+  auto part_at = [&](int g, int q) __attribute__((always_inline)) {
+    return lds_ptr<float4>(lds0 + g * P::kArea + (kShare == 1 ? q : cg) * kPartBytes);
+  };
+  auto ml_at = [&](int g) __attribute__((always_inline)) {
+    return lds_ptr<float>(lds0 + g * P::kArea + (kShare == 1 ? g * kPartBytes : 2 * kPartBytes + cg * 1024u));
+  };
+  static_for<NB>([&](auto bc) __attribute__((always_inline)) {
+    constexpr int b = bc;
+    if (b != 0) __syncthreads(); // block b - 1 has been merged
+    floatx16 f[P::kParts]; // this wave's share of its own part
+#pragma unroll
+    for (int j = 0; j < P::kParts; ++j) f[j] = floatx16{};
+    acc_fence();
+    static_for<KS>([&](auto q) __attribute__((always_inline)) {
+      constexpr int r0 = 16 * (8 * b + P::kParts * q);
+      if (q != kg) {
+        float4 *to = part_at(kg, q);
+        static_for<4 * P::kParts>([&](auto ji) __attribute__((always_inline)) {
+          constexpr int r = r0 + 4 * ji;
+          to[kWave * ji + lane_e] = make_float4(acc_get<r>(), acc_get<r + 1>(), acc_get<r + 2>(), acc_get<r + 3>());
+        });
+      } else {
+        static_for<16 * P::kParts>([&](auto i) __attribute__((always_inline)) { f[i / 16][i % 16] = acc_get<r0 + i>(); });
+      }
+    });
+    acc_fence();
+    if (b == 0) {
+#pragma unroll
+      for (int bb = 0; bb < NB; ++bb) {
+        ml_at(kg)[(2 * bb) * kWave + lane_e] = m_run[bb];
+        ml_at(kg)[(2 * bb + 1) * kWave + lane_e] = l_run[bb];
+      }
+      wait_vm<0>(); // this wave's gate rows
+    }
+    __syncthreads();
+    // The gate pieces of this lane (its column's row, dims 8 k + 4 half .. +3 of
+    // the part), read before the partials so that no round trip waits for another.
+    constexpr int kChunks = 4 * P::kParts; // 16-byte chunks of a row's part
+    const int r0 = 32 * (NB * cg + b);
+    const unsigned row = row_at(r0 + col_e);
+    auto gate_at = [&](int k) __attribute__((always_inline)) {
+      return row + 16u * ((kChunks * kg + k) ^ swz(col_e)) + 8u * half_e;
+    };
+    u32x2 gp[kChunks];
+#pragma unroll
+    for (int k = 0; k < kChunks; ++k) gp[k] = *lds_ptr<u32x2>(gate_at(k));
+    float mw[KS], lw[KS], mm = -INFINITY, lsum = 0.f;
+#pragma unroll
+    for (int g = 0; g < KS; ++g) {
+      mw[g] = ml_at(g)[(2 * b) * kWave + lane_e];
+      lw[g] = ml_at(g)[(2 * b + 1) * kWave + lane_e];
+    }
+#pragma unroll
+    for (int g = 0; g < KS; ++g) mm = fmaxf(mm, mw[g]);
+#pragma unroll
+    for (int g = 0; g < KS; ++g) {
+      mw[g] = fexp2(mw[g] - mm); // a wave that saw no key has m = -inf and weight 0
+      lsum += mw[g] * lw[g];
+    }
+    const float a_own = fexp2(m_run[b] - mm);
+#pragma unroll
+    for (int j = 0; j < P::kParts; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) f[j][i] *= a_own;
+#pragma unroll
+    for (int g = 0; g < KS; ++g) {
+      if (g == kg) continue;
+      const float4 *from = part_at(g, kg);
+#pragma unroll
+      for (int j = 0; j < P::kParts; ++j)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const float4 x = from[kWave * (4 * j + i4) + lane_e];
+          f[j][4 * i4] += mw[g] * x.x;
+          f[j][4 * i4 + 1] += mw[g] * x.y;
+          f[j][4 * i4 + 2] += mw[g] * x.z;
+          f[j][4 * i4 + 3] += mw[g] * x.w;
+        }
+    }
+    const float inv = 1.0f / (lsum + xor32(lsum));
+    // The gate pieces become the gated outputs, which leave as whole lines.
+#pragma unroll
+    for (int j = 0; j < P::kParts; ++j)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4) {
+        const u32x2 g = gp[4 * j + i4];
+        const floatx16 &x = f[j];
+        gp[4 * j + i4] = u32x2{pack_bf16x2(x[4 * i4] * inv * sigmoid_gate(bf16_lo(g[0])),
+                                           x[4 * i4 + 1] * inv * sigmoid_gate(bf16_hi(g[0]))),
+                               pack_bf16x2(x[4 * i4 + 2] * inv * sigmoid_gate(bf16_lo(g[1])),
+                                           x[4 * i4 + 3] * inv * sigmoid_gate(bf16_hi(g[1])))};
+      }
+#pragma unroll
+    for (int k = 0; k < kChunks; ++k) *lds_ptr<u32x2>(gate_at(k)) = gp[k];
+    wave_lds_order(); // the rows' pieces are read back by other lanes of this wave
+    constexpr int kPerStore = kWave / kChunks; // rows
+#pragma unroll
+    for (int i = 0; i < 32 / kPerStore; ++i) {
+      const int c = kPerStore * i + lane_e / kChunks, k = kChunks * kg + lane_e % kChunks, r = r0 + c;
+      if (static_cast<std::size_t>(8 * (r >> 5) + (r & 7)) < q_rows)
+        *reinterpret_cast<u32x4 *>(output + io_row(r) + 8 * k) = *lds_ptr<u32x4>(row_at(r) + 16u * (k ^ swz(c)));
+    }
+  });
+  if constexpr (FromInput) {
+#pragma unroll
+    for (int j = 0; j < kApp; ++j) {
+      int pl, tok, piece;
+      app_at(j, pl, tok, piece);
+      if (static_cast<std::size_t>(tok) < q_rows)
+        *reinterpret_cast<u32x4 *>(cache + pl * plane + cache_row(HeadMajor, t0 + tok, kv_head, max_ctx) + 8 * piece) =
+            app[j];
+    }
+  }
+}
+
+template <int NB, int KS>
+void launch(const bf16_bits *q, const bf16_bits *key, const bf16_bits *value, const bf16_bits *gate, bf16_bits *out,
+            bf16_bits *cache, std::size_t tokens, std::size_t max_ctx, std::size_t past, bool head_major,
+            bool fused_append, const PrefillNormRope *nq, hipStream_t stream) {
+  // 8 workgroups (one per XCD) per pair of query tiles
+  const unsigned grid =
+      static_cast<unsigned>(8 * ceil_div_unchecked(ceil_div_unchecked(tokens, Plan<NB, KS>::kTok), 2));
+  const PrefillNormRope arg = nq != nullptr ? *nq : PrefillNormRope{};
+  auto go = [&](auto kernel) {
+    kernel<<<grid, kThreads, 0, stream>>>(q, key, value, gate, out, cache, tokens, max_ctx, past, arg);
+  };
+  if (nq != nullptr)
+    go(head_major ? prefill_wide_kernel<NB, KS, true, false, true> : prefill_wide_kernel<NB, KS, false, false, true>);
+  else if (fused_append)
+    go(head_major ? prefill_wide_kernel<NB, KS, true, true, false> : prefill_wide_kernel<NB, KS, false, true, false>);
+  else
+    go(head_major ? prefill_wide_kernel<NB, KS, true, false, false> : prefill_wide_kernel<NB, KS, false, false, false>);
+}
+} // namespace
+
+void launch_prefill_wide(PrefillForm form, const bf16_bits *q, const bf16_bits *key, const bf16_bits *value,
+                         const bf16_bits *gate, bf16_bits *out, bf16_bits *cache, std::size_t tokens,
+                         std::size_t max_ctx, std::size_t past, bool head_major, bool fused_append,
+                         const prefill::PrefillNormRope *nq, hipStream_t stream) {
+  switch (form) {
+  case PrefillForm::stream8:
+    return launch<1, 4>(q, key, value, gate, out, cache, tokens, max_ctx, past, head_major, fused_append, nq, stream);
+  case PrefillForm::stream16:
+    return launch<2, 4>(q, key, value, gate, out, cache, tokens, max_ctx, past, head_major, fused_append, nq, stream);
+  default:
+    return launch<2, 2>(q, key, value, gate, out, cache, tokens, max_ctx, past, head_major, fused_append, nq, stream);
+  }
+}
+
+} // namespace raftinfer::amd

@@ -31,4 +31,21 @@ void launch_prefill_mfma_fused(const bf16_bits *query_gate, const bf16_bits *key
                                bool weight_f32, int pairs, double ratio, float epsilon,
                                hipStream_t stream);
 
+// How a prefill call is split (prefill_plan): prefill_mfma_kernel with 8 query
+// tokens per workgroup, or the streaming kernel of attention_prefill_wide.hip
+// with 8, 16 or 32.
+enum class PrefillForm { short8, stream8, stream16, stream32 };
+PrefillForm prefill_plan(std::size_t tokens, std::size_t past);
+
+namespace prefill {
+struct PrefillNormRope;
+}
+// The streaming forms; the same requirements.  With nq != nullptr q is the raw q
+// projection (gate, key and value are not read) and the cache holds every key.
+void launch_prefill_wide(PrefillForm form, const bf16_bits *q, const bf16_bits *key,
+                         const bf16_bits *value, const bf16_bits *gate, bf16_bits *out,
+                         bf16_bits *cache, std::size_t tokens, std::size_t max_ctx,
+                         std::size_t past, bool head_major, bool fused_append,
+                         const prefill::PrefillNormRope *nq, hipStream_t stream);
+
 } // namespace raftinfer::amd

@@ -42,9 +42,28 @@ def test_compiler_mfmas_and_mfma_chains_are_not_flagged():
     assert asm_mfma_hazards(text) == []
 
 
+def test_vector_results_operand_writes_and_owned_registers():
+    mfma = MFMA.replace("\ts_nop 1\n", "").replace("a[16:31]", "v[40:55]")
+    for line in ("\tv_mov_b32_e32 v1, v41\n", "\tv_mov_b32_e32 v55, v1\n", "\tds_write_b32 v1, v50\n"):
+        assert len(asm_mfma_hazards(mfma + line)) == 1, line
+        assert asm_mfma_hazards(mfma + "\ts_nop 7\n" * 3 + line) == [], line
+    # an operand written by the vector unit right before, then two wait states before
+    write = "\tv_add_f32_e32 v32, v1, v2\n"
+    assert len(asm_mfma_hazards(write + "\ts_nop 0\n" + mfma)) == 1
+    assert asm_mfma_hazards(write + "\ts_nop 1\n" + mfma) == []
+    # registers named in hexadecimal, and the rule for kernels that own the accumulation registers
+    assert len(asm_mfma_hazards(MFMA.replace("a[16:31]", "a[0x80:0x8f]") + "\tv_accvgpr_read_b32 v0, a[0x81]\n")) == 1
+    spill = "\tv_accvgpr_write_b32 a3, v9\n"
+    assert asm_mfma_hazards(spill) == []
+    assert len(asm_mfma_hazards(spill, owned_agprs=True)) == 1
+    assert asm_mfma_hazards("\t;;#ASMSTART\n" + spill + "\t;;#ASMEND\n", owned_agprs=True) == []
+
+
 def test_built_prefill_kernel_has_no_hazard():
     s = pathlib.Path(asm_check.__file__).resolve().parent / "_build" / "attention_prefill_mfma.hip.s"
     if not s.exists():
         import pytest
         pytest.skip("the library has not been built here")
     assert asm_mfma_hazards(s.read_text()) == []
+    wide = s.with_name("attention_prefill_wide.hip.s")
+    assert asm_mfma_hazards(wide.read_text(), owned_agprs=True) == []
