@@ -351,13 +351,13 @@ void launch_prefill(const void *q, const void *k, const void *v, const void *g, 
   const std::size_t kv_elements = s.tokens * s.kv_heads * s.head_dim;
   const int append_grid = static_cast<int>(ceil_div_unchecked(kv_elements, kBlockSize));
   bool mfma = false, fused = false;
-  if constexpr (std::is_same_v<ActT, bf16_bits> && std::is_same_v<CacheT, bf16_bits>) {
+  if constexpr (std::is_same_v<ActT, bf16_bits>) {
     const auto bits = [](const void *p) { return reinterpret_cast<std::uintptr_t>(p); };
     mfma = ((bits(q) | bits(cache)) & 15u) == 0 && ((bits(g) | bits(o)) & 7u) == 0 &&
            s.query_heads == kQueryHeads && s.kv_heads == kKvHeads && s.head_dim == kHeadDim;
     // A prompt with no past reads its keys straight from key/value and
     // appends them inside the attention kernel.
-    fused = mfma && s.past_tokens == 0 && ((bits(k) | bits(v)) & 15u) == 0;
+    fused = mfma && std::is_same_v<CacheT, bf16_bits> && s.past_tokens == 0 && ((bits(k) | bits(v)) & 15u) == 0;
   }
   if (!kernel_only && !fused) {
     append_prefill_kernel<ActT, CacheT><<<append_grid, kBlockSize, 0, stream>>>(
@@ -372,6 +372,12 @@ void launch_prefill(const void *q, const void *k, const void *v, const void *g, 
                                static_cast<bf16_bits *>(o), static_cast<bf16_bits *>(cache), s.tokens,
                                s.max_context_tokens, s.past_tokens, head_major, fused, stream);
       check_launch<Err>("qwen35_online_attention_prefill_gfx950_mfma_hd256");
+      return;
+    } else if constexpr (std::is_same_v<ActT, bf16_bits>) {
+      amd::launch_prefill_f32_cache(static_cast<const bf16_bits *>(q), static_cast<const bf16_bits *>(g),
+                                    static_cast<bf16_bits *>(o), static_cast<float *>(cache), s.tokens,
+                                    s.max_context_tokens, s.past_tokens, head_major, stream);
+      check_launch<Err>("qwen35_online_attention_prefill_gfx950_mfma_f32_cache");
       return;
     }
   }

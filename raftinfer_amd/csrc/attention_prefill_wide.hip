@@ -28,6 +28,7 @@
 #include "prefill_mfma.hpp"
 #include "prefill_tile.hpp"
 
+#include <type_traits>
 #include <utility>
 
 namespace raftinfer::amd {
@@ -138,12 +139,43 @@ template <int NB, int KS> struct Plan {
   static constexpr int kParts = 8 / KS;                 // dims blocks that a wave finishes
 };
 
-template <int NB, int KS, bool HeadMajor, bool FromInput, bool NormQ>
+// ---- f32 cache (F32).  K, V, the probabilities and all sums stay f32: f32 MFMAs
+// have a sixteenth of the bf16 rate, so a value is split into three bf16 parts of
+// 8 bits (x = h + m + l exactly, by truncation), and the products of parts that
+// matter at f32 precision are summed in f32.  Cache rows appended from bf16
+// activations have m = l = 0; each half tile is checked, and takes the products
+// with m and l only if some value has more bits.  A tile is 16 keys, so its halves
+// are the same 8 KiB ring items; S and PV are not overlapped.  The vector unit
+// bounds it (the checks and packing of 8192 values per wave and tile).  512 tokens
+// on a token-major f32 cache: 866 us with one wave per row and fp32 FMAs, now 31.
+__device__ __forceinline__ std::uint32_t high_pair(float a, float b) { // truncated bf16 of (a, b)
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+// What x - h is; 0 for an infinity.
+__device__ __forceinline__ float rest_part(float x) {
+  const float h = __uint_as_float(__float_as_uint(x) & 0xFFFF0000u);
+  return __builtin_isinf(x) ? 0.f : x - h;
+}
+__device__ __forceinline__ bf16x8 high_operand(const float (&x)[8]) {
+  return __builtin_bit_cast(bf16x8, u32x4{high_pair(x[0], x[1]), high_pair(x[2], x[3]), high_pair(x[4], x[5]),
+                                          high_pair(x[6], x[7])});
+}
+__device__ __forceinline__ floatx4 lds_read_f4(unsigned addr) {
+  return *(const __attribute__((address_space(3))) floatx4 *)(std::uintptr_t)(addr);
+}
+__device__ __forceinline__ float lds_read_f1(unsigned addr) {
+  return *(const __attribute__((address_space(3))) float *)(std::uintptr_t)(addr);
+}
+template <bool F32> using CacheElem = std::conditional_t<F32, float, bf16_bits>;
+
+template <int NB, int KS, bool HeadMajor, bool FromInput, bool NormQ, bool F32 = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_wide_kernel(
     const bf16_bits *__restrict__ query, const bf16_bits *key_in, const bf16_bits *value_in,
-    const bf16_bits *gate, bf16_bits *__restrict__ output, bf16_bits *__restrict__ cache,
+    const bf16_bits *gate, bf16_bits *__restrict__ output, CacheElem<F32> *__restrict__ cache,
     std::size_t tokens, std::size_t max_ctx, std::size_t past, PrefillNormRope nq) {
   static_assert(!(NormQ && FromInput), "the fused producer path reads K/V from the cache");
+  static_assert(!F32 || (NB == 1 && KS == 4 && !FromInput && !NormQ), "the form of the f32 cache");
+  constexpr int kTileKeys = F32 ? 16 : kKTile;
   using P = Plan<NB, KS>;
   constexpr int kTok = P::kTok, kShare = P::kShare;
   constexpr unsigned kSlot = P::kSlot;
@@ -161,7 +193,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   const std::size_t t0 = qtile * kTok;
   const std::size_t q_rows = tokens - t0 < kTok ? tokens - t0 : kTok;
   const std::size_t key_end = past + t0 + q_rows;
-  const std::size_t n_tiles = (key_end + kKTile - 1) / kKTile;
+  const std::size_t n_tiles = (key_end + kTileKeys - 1) / kTileKeys;
   const std::size_t plane = max_ctx * kKvHeads * kHeadDim;
   const float scale = kLog2e / 16.0f;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -200,10 +232,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   // The 16 rows of a ds_read_b128 pass over K then share no bank, nor do the 4
   // rows x 64 bytes of a ds_read_b64_tr_b16 pass over V, whose rows 8 apart have
   // the same f.  A load's offset is the lane's, an exclusive-or and an addition.
-  constexpr std::uint32_t row_bytes = HeadMajor && !FromInput ? kHeadDim * 2 : kKvHeads * kHeadDim * 2;
-  const bf16_bits *k_src = FromInput ? key_in + kv_head * kHeadDim
-                                     : cache + cache_row(HeadMajor, 0, kv_head, max_ctx);
-  const bf16_bits *v_src = FromInput ? value_in + kv_head * kHeadDim : k_src + plane;
+  constexpr std::uint32_t row_bytes =
+      (HeadMajor && !FromInput ? kHeadDim : kKvHeads * kHeadDim) * sizeof(CacheElem<F32>);
+  const CacheElem<F32> *k_src, *v_src;
+  if constexpr (FromInput) {
+    k_src = key_in + kv_head * kHeadDim;
+    v_src = value_in + kv_head * kHeadDim;
+  } else {
+    k_src = cache + cache_row(HeadMajor, 0, kv_head, max_ctx);
+    v_src = k_src + plane;
+  }
   constexpr int k_rows = kShare == 1 ? 4 : 2; // rows per K load
   const int hrow = kShare == 1 ? lane >> 4 : half;
   const std::uint32_t v_off = half * row_bytes + 16u * (col ^ (8 * half));
@@ -218,13 +256,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     load_lds_b128_at<1024 * (i & 3)>(base + 4096 * (i >> 2), load_offset<64u * (i & 1), i *(2 * row_bytes - 1024)>(v_off),
                                      to + 4096u * (i >> 2));
   };
-  auto base_of = [&](const bf16_bits *src, std::size_t row) __attribute__((always_inline)) {
+  auto base_of = [&](const CacheElem<F32> *src, std::size_t row) __attribute__((always_inline)) {
     return reinterpret_cast<const unsigned char *>(src) + row * row_bytes;
   };
   // The same for items that may reach past key_end: those rows re-read the last
   // one (their scores are masked).  k0: first row; for K of own tiles `half_tile`
   // is the dims half.
-  auto load_clamped = [&](const bf16_bits *src, auto is_v, std::size_t k0, int half_tile, unsigned to, auto ic)
+  auto load_clamped = [&](const CacheElem<F32> *src, auto is_v, std::size_t k0, int half_tile, unsigned to, auto ic)
       __attribute__((always_inline)) {
     constexpr int i = ic;
     constexpr bool dims_half = kShare == 1 && !is_v;
@@ -242,11 +280,25 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   // Tile of this wave's key group, counted from its first, and the first row of
   // its share `sub` of it.
   auto tile_row = [&](std::size_t n, int sub) __attribute__((always_inline)) {
-    return (n * KS + kg) * kKTile + 16 * sub;
+    return (n * KS + kg) * kTileKeys + 16 * sub;
   };
   constexpr std::false_type kIsK{};
   constexpr std::true_type kIsV{};
-  auto load_item = [&](const bf16_bits *src, auto is_v, std::size_t k0, int half_tile, unsigned to)
+  // An f32 half tile (16 rows of 128 dims, two rows a load): chunk c (0..31) at
+  // c ^ row for K (a ds_read_b128 pass takes one chunk of 16 rows), at c ^ 8
+  // (row / 4 % 2) for V (a ds_read_b32 takes 32 dims of two rows 4 apart).
+  auto load_f32 = [&](bool is_v, std::size_t tile, int hh, unsigned to) __attribute__((always_inline)) {
+    const std::size_t k0 = (tile * KS + kg) * kTileKeys;
+    const int l = late_lane();
+    const std::uint32_t last = static_cast<std::uint32_t>(key_end - 1 - k0 < 15 ? key_end - 1 - k0 : 15);
+    const unsigned char *base = base_of(is_v ? v_src : k_src, k0) + 512 * hh;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const std::uint32_t r = 2 * i + (l >> 5), f = is_v ? 8 * ((i >> 1) & 1) : r;
+      load_lds_b128_at<0>(base, (r < last ? r : last) * row_bytes + 16u * ((l & 31) ^ f), to + 1024u * i);
+    }
+  };
+  auto load_item = [&](const CacheElem<F32> *src, auto is_v, std::size_t k0, int half_tile, unsigned to)
       __attribute__((always_inline)) {
     static_for<8>([&](auto i) __attribute__((always_inline)) { load_clamped(src, is_v, k0, half_tile, to, i); });
   };
@@ -277,7 +329,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   const int my = kShare > 1 ? cg : 0; // this wave's share of an item
   const unsigned part = 8192u * my;
   auto issue_start = [&](int from, int to) __attribute__((always_inline)) {
-    if constexpr (kShare == 1) {
+    if constexpr (F32) { // K0 K1 V0 V1 of tile 0
+      for (int n = from; n < to; ++n)
+        if (m != 0) load_f32(n >= 2, 0, n & 1, ring + n * kSlot);
+    } else if constexpr (kShare == 1) {
       for (int n = from; n < to; ++n)
         if (static_cast<std::size_t>(n >> 1) < m) load_item(k_src, kIsK, tile_row(n >> 1, 0), n & 1, ring + n * kSlot);
     } else {
@@ -342,7 +397,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   }
   if constexpr (!NormQ) {
     // this wave's Q rows have landed, then every other wave's
-    if constexpr (kShare == 1) {
+    if constexpr (F32) {
+      if (m != 0) wait_vm<32>(); else wait_vm<0>();
+    } else if constexpr (kShare == 1) {
       if (m > 1) wait_vm<32>(); else if (m != 0) wait_vm<16>(); else wait_vm<0>();
     } else {
       if (m > 1) wait_vm<24>(); else wait_vm<16>();
@@ -609,7 +666,178 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     }
     ++n;
   };
-  if (m != 0) {
+  if constexpr (F32) {
+    // Ring items K0 K1 V0 V1 of one tile after the other; while item n is read,
+    // n + 4 (the same part of the next tile) is loaded into the slot of n - 1.
+    const int row = lane & 15;
+    const bool low = (lane & 16) != 0;
+    const unsigned kf_lane = row * 512u + 16u * ((2 * half) ^ row);
+    const unsigned vf_lane = half * 2048u + 128u * half + 4u * col;
+    for (; n < m; ++n) {
+      const bool more = n + 1 < m;
+      auto next_item = [&](bool is_v, int hh, int left) __attribute__((always_inline)) {
+        if (more || left == 3) wait_vm<24>(); else if (left == 2) wait_vm<16>(); else if (left == 1) wait_vm<8>(); else wait_vm<0>();
+        if (more) load_f32(is_v, n + 1, hh, p0);
+      };
+      // S^T: A rows r and r + 16 both hold key r.  High parts first (rows 16..
+      // repeat them and are not used); if some value has more bits, rows 0..15
+      // the middle and rows 16.. the low parts into a second accumulator.
+      floatx16 sm = floatx16{};
+      bool rest = false;
+      static_for<2>([&](auto hh) __attribute__((always_inline)) {
+        next_item(false, hh, 3 - hh);
+        const unsigned a0 = p1 + kf_lane;
+        auto values = [&](unsigned base, int kk, float(&y)[8]) __attribute__((always_inline)) { // kk in the half
+          const unsigned a = (base ^ (64u * (kk & 3))) + 256u * (kk >> 2);
+          const floatx4 u = lds_read_f4(a), w = lds_read_f4(a ^ 16u);
+          y[0] = u[0]; y[1] = u[1]; y[2] = u[2]; y[3] = u[3];
+          y[4] = w[0]; y[5] = w[1]; y[6] = w[2]; y[7] = w[3];
+        };
+        std::uint32_t bits = 0;
+        float y[4][8];
+        static_for<4>([&](auto j) __attribute__((always_inline)) { values(a0, j, y[j]); });
+        static_for<8>([&](auto kk) __attribute__((always_inline)) {
+          float(&v)[8] = y[kk & 3];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) bits |= __float_as_uint(v[j]);
+          bf16x8 a = high_operand(v);
+          asm volatile("s_nop 1" : "+v"(a)); // (wait states before the MFMA)
+          if constexpr (hh == 0 && kk == 0) s_mfma_zero(s0[0], a, qa[0][0]); else s_mfma(s0[0], a, qa[0][8 * hh + kk]);
+          if constexpr (kk < 4) values(a0, kk + 4, y[kk & 3]);
+          __builtin_amdgcn_sched_barrier(0);
+        });
+        if (__builtin_amdgcn_ballot_w64((bits & 0xFFFFu) != 0) != 0) {
+          rest = true;
+          static_for<8>([&](auto kk) __attribute__((always_inline)) {
+            float v[8];
+            values(a0, kk, v);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              v[j] = rest_part(v[j]);
+              v[j] = low ? rest_part(v[j]) : v[j];
+            }
+            bf16x8 a = high_operand(v);
+            asm volatile("s_nop 1" : "+v"(a), "+v"(sm));
+            s_mfma(sm, a, qa[0][8 * hh + kk]);
+            __builtin_amdgcn_sched_barrier(0);
+          });
+        }
+        advance(1);
+      });
+      asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(s0[0]), "+v"(sm));
+      float x[8]; // scores, then probabilities, of keys 4 half + 0..3 and 8 + 4 half + 0..3
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = s0[0][i];
+      if (rest)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] += sm[i] + sm[8 + i];
+      const std::ptrdiff_t rel = static_cast<std::ptrdiff_t>(past + t0 + slot_row(col)) -
+                                 static_cast<std::ptrdiff_t>(tile_row(n, 0));
+      const int lim = rel < -1 ? -1 : (rel > kTileKeys ? kTileKeys : static_cast<int>(rel)); // last visible key
+      float mxs = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        x[i] = (i >> 2) * 8 + 4 * half + (i & 3) > lim ? -INFINITY : x[i] * scale;
+        mxs = fmaxf(mxs, x[i]);
+      }
+      mxs = max_xor32(mxs);
+      const bool grow = mxs > m_run[0] + kLazyRescale;
+      if (n == 0) {
+        m_run[0] = grow ? mxs : m_run[0];
+      } else if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+        mfma_drain();
+        const float sc = grow ? fexp2(m_run[0] - mxs) : 1.0f;
+        l_run[0] *= sc;
+        m_run[0] = grow ? mxs : m_run[0];
+        static_for<128>([&](auto r) __attribute__((always_inline)) { acc_set<r>(acc_get<r>() * sc); });
+      }
+      const float mref = m_run[0] == -INFINITY ? 0.f : m_run[0];
+      float pr[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        x[i] = fexp2(x[i] - mref);
+        l_run[0] += x[i];
+        pr[i] = rest_part(x[i]);
+      }
+      const bf16x8 ph = high_operand(x), pm = high_operand(pr);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) pr[i] = rest_part(pr[i]);
+      const bf16x8 pl = high_operand(pr);
+      // O^T += V^T P^T, 4 dims blocks per half tile.
+      static_for<2>([&](auto hh) __attribute__((always_inline)) {
+        next_item(true, hh, 1 - hh);
+        acc_fence();
+        const unsigned a0 = p1 + vf_lane;
+        auto values = [&](int nb, float(&y)[8]) __attribute__((always_inline)) { // dim 32 nb + col of the half
+#pragma unroll
+          for (int i = 0; i < 8; ++i) y[i] = lds_read_f1((a0 ^ (128u * nb)) + 512u * (8 * (i >> 2) + (i & 3)));
+        };
+        std::uint32_t bits = 0;
+        float finite = 0.f; // NaN if some value is an infinity or a NaN
+        bf16x8 vh[4];
+        static_for<4>([&](auto nb) __attribute__((always_inline)) {
+          float y[8];
+          values(nb, y);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            bits |= __float_as_uint(y[i]);
+            finite = fmaf(y[i], 0.f, finite);
+          }
+          vh[nb] = high_operand(y);
+        });
+        if (__builtin_amdgcn_ballot_w64(finite != finite) != 0) {
+          // key by key: a zero part of a probability times an infinity is not 0,
+          // and a masked key must not count
+          mfma_drain();
+#pragma unroll 1
+          for (int key = 0; key < kTileKeys; ++key) {
+            float w = x[0]; // the key's probability, in the lanes of its half, then in the whole column
+#pragma unroll
+            for (int i = 1; i < 8; ++i) {
+              w = i == 4 * (key >> 3) + (key & 3) ? x[i] : w;
+              asm volatile("" : "+v"(w)); // a chain of selects, not an array in scratch
+            }
+            const float other = xor32(w);
+            w = ((key >> 2) & 1) != half ? other : w;
+            const unsigned a = p1 + key * 512u;
+            static_for<64>([&](auto r) __attribute__((always_inline)) {
+              constexpr int i = r & 15, d = 32 * (r >> 4) + 8 * (i >> 2) + (i & 3); // + 4 half
+              const float y = lds_read_f1(a + 16u * ((((d + 4 * half) >> 2)) ^ (8 * ((key >> 2) & 1))) + 4u * (d & 3));
+              const float was = acc_get<64 * hh + r>();
+              acc_set<64 * hh + r>(key <= lim ? fmaf(w, y, was) : was);
+            });
+            acc_fence();
+          }
+        } else {
+          // the smallest products first
+          asm volatile("s_nop 1" : "+v"(vh[0]), "+v"(vh[1]), "+v"(vh[2]), "+v"(vh[3]));
+          static_for<4>([&](auto nb) __attribute__((always_inline)) { acc_mfma<4 * hh + nb>(vh[nb], pl); });
+          static_for<4>([&](auto nb) __attribute__((always_inline)) { acc_mfma<4 * hh + nb>(vh[nb], pm); });
+          static_for<4>([&](auto nb) __attribute__((always_inline)) { acc_mfma<4 * hh + nb>(vh[nb], ph); });
+          if (__builtin_amdgcn_ballot_w64((bits & 0xFFFFu) != 0) != 0) {
+            static_for<4>([&](auto nb) __attribute__((always_inline)) {
+              float y[8];
+              values(nb, y);
+#pragma unroll
+              for (int i = 0; i < 8; ++i) y[i] = rest_part(y[i]);
+              bf16x8 vm = high_operand(y);
+#pragma unroll
+              for (int i = 0; i < 8; ++i) y[i] = rest_part(y[i]);
+              bf16x8 vl = high_operand(y);
+              asm volatile("s_nop 1" : "+v"(vm), "+v"(vl));
+              acc_mfma<4 * hh + nb>(vl, ph);
+              acc_mfma<4 * hh + nb>(vm, pm);
+              acc_mfma<4 * hh + nb>(vm, ph);
+            });
+          }
+        }
+        acc_fence();
+        advance(1);
+      });
+    }
+    mfma_drain();
+    wait_lgkm0();
+  } else if (m != 0) {
     // S of the first tile: items 0, 1 (own) or 0 (shared) are read, V(0) or K(2) loaded.
     if constexpr (kShare == 1) {
       if (m > 1) wait_vm<24>(); else wait_vm<8>(); // K(0), first half
@@ -819,6 +1047,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   }
 }
 
+void launch_f32(const bf16_bits *q, const bf16_bits *gate, bf16_bits *out, float *cache, std::size_t tokens,
+                std::size_t max_ctx, std::size_t past, bool head_major, hipStream_t stream) {
+  const unsigned grid = static_cast<unsigned>(8 * ceil_div_unchecked(ceil_div_unchecked(tokens, Plan<1, 4>::kTok), 2));
+  auto go = [&](auto kernel) {
+    kernel<<<grid, kThreads, 0, stream>>>(q, nullptr, nullptr, gate, out, cache, tokens, max_ctx, past,
+                                          PrefillNormRope{});
+  };
+  go(head_major ? prefill_wide_kernel<1, 4, true, false, false, true>
+                : prefill_wide_kernel<1, 4, false, false, false, true>);
+}
+
 template <int NB, int KS>
 void launch(const bf16_bits *q, const bf16_bits *key, const bf16_bits *value, const bf16_bits *gate, bf16_bits *out,
             bf16_bits *cache, std::size_t tokens, std::size_t max_ctx, std::size_t past, bool head_major,
@@ -838,6 +1077,12 @@ void launch(const bf16_bits *q, const bf16_bits *key, const bf16_bits *value, co
     go(head_major ? prefill_wide_kernel<NB, KS, true, false, false> : prefill_wide_kernel<NB, KS, false, false, false>);
 }
 } // namespace
+
+void launch_prefill_f32_cache(const bf16_bits *q, const bf16_bits *gate, bf16_bits *out, float *cache,
+                              std::size_t tokens, std::size_t max_ctx, std::size_t past, bool head_major,
+                              hipStream_t stream) {
+  launch_f32(q, gate, out, cache, tokens, max_ctx, past, head_major, stream);
+}
 
 void launch_prefill_wide(PrefillForm form, const bf16_bits *q, const bf16_bits *key, const bf16_bits *value,
                          const bf16_bits *gate, bf16_bits *out, bf16_bits *cache, std::size_t tokens,

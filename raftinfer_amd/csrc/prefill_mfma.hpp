@@ -16,6 +16,12 @@ void launch_prefill_mfma(const bf16_bits *q, const bf16_bits *key, const bf16_bi
                          std::size_t tokens, std::size_t max_ctx, std::size_t past,
                          bool head_major, bool fused_append, hipStream_t stream);
 
+// The same with an f32 cache, used at full precision; the cache must already hold
+// positions 0..past+tokens-1.
+void launch_prefill_f32_cache(const bf16_bits *q, const bf16_bits *gate, bf16_bits *out,
+                              float *cache, std::size_t tokens, std::size_t max_ctx,
+                              std::size_t past, bool head_major, hipStream_t stream);
+
 // The producers fused in (query_gate: the raw q projection [tokens][16][2][256];
 // key: the raw k projection [tokens][4][256]): a key kernel normalises and
 // rotates k and appends k and v at positions past..past+tokens-1, then the

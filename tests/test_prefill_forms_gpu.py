@@ -84,3 +84,94 @@ def test_streaming_forms_fused_equal_producers_then_attention(gpu, T, past, rot,
     c = _prefill_case(T, past, rot, wdt, layout, seed=T + past)
     assert torch.equal(c["cache1"], c["cache2"])
     assert torch.equal(c["out1"], c["out2"])
+
+
+# ---- the f32 cache at the model shape (K, V and the probabilities at f32 precision; tiles of 16 keys, a round of 64)
+def f32_cache(T, past, layout, seed, exact_bf16=False, edit=None):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *shape: torch.randn(*shape, device="cuda", generator=g)
+    n = past + T
+    q, gate = rnd(T, HQ, D).bfloat16(), rnd(T, HQ, D).bfloat16()
+    rows = rnd(2, n, HKV, D)
+    if exact_bf16:
+        rows = rows.bfloat16().float()
+    rows[:, past:] = rows[:, past:].bfloat16().float()
+    if edit is not None:
+        edit(rows)
+    cache = rows.clone()
+    cache[:, past:] = 0
+    cache = (cache.transpose(1, 2) if layout == 1 else cache).contiguous()
+    out = torch.empty(T, HQ, D, device="cuda", dtype=torch.bfloat16)
+    ops.qwen35_causal_attention(q, rows[0, past:].bfloat16(), rows[1, past:].bfloat16(), gate, out, cache, None,
+                                S(T, HQ, HKV, D, n, past), 3, ops.Qwen35AttentionLaunchPolicy(1, 0, layout))
+    torch.cuda.synchronize()
+    kf, vf = (x.double().repeat_interleave(HQ // HKV, dim=1).permute(1, 0, 2).contiguous() for x in rows)
+    s = torch.matmul(q.double().permute(1, 0, 2), kf.transpose(1, 2).contiguous()) / 16.0
+    hidden = torch.arange(n, device="cuda")[None] > past + torch.arange(T, device="cuda")[:, None]
+    p = torch.softmax(s.masked_fill(hidden, float("-inf")), dim=-1)
+    written = cache if layout == 0 else cache.transpose(1, 2)
+    return out, p, vf, gate.double(), hidden, torch.equal(written, rows)
+
+
+@pytest.mark.parametrize("T,past", [(2, 0), (9, 7), (16, 0), (17, 15), (65, 0), (64, 63), (100, 333), (512, 512)])
+@pytest.mark.parametrize("layout,exact_bf16", [(0, True), (1, False), (0, False)])
+def test_f32_cache_prefill(gpu, T, past, layout, exact_bf16):
+    out, p, v, gate, _, same = f32_cache(T, past, layout, seed=T + past, exact_bf16=exact_bf16)
+    assert same, "appended rows"
+    want = (torch.matmul(p, v).permute(1, 0, 2) * torch.sigmoid(gate)).cpu().numpy()
+    got = from_dev(out)
+    # f32 sums of about 1e-6 of the largest product each, then one rounding to bf16 (2^-8 of the value at most)
+    assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) * 1.001 + 2e-5)
+
+
+def test_f32_cache_prefill_keeps_bits_below_bf16(gpu):
+    # Keys that differ only below bf16 decide the result: scores 1000 (1 + 2^-12 j) have softmax steps of 0.24 in j,
+    # and in bf16 they would all be 1000.  V is the position, so the output is the mean position.
+    T, n = 2, 40
+    past = n - T
+    rows = torch.zeros(2, n, HKV, D, device="cuda")
+    j = torch.arange(past, device="cuda", dtype=torch.float32)
+    rows[0, :past, :, 0] = (1000.0 * (1 + j * 2.0 ** -12))[:, None]
+    rows[1, :past] = (j / past)[:, None, None]
+    q = torch.zeros(T, HQ, D, device="cuda", dtype=torch.bfloat16)
+    q[:, :, 0] = 16.0  # score = q.k / 16 = k[0]
+    out = torch.empty(T, HQ, D, device="cuda", dtype=torch.bfloat16)
+    zero = torch.zeros(T, HKV, D, device="cuda", dtype=torch.bfloat16)
+    ops.qwen35_causal_attention(q, zero, zero, torch.zeros_like(q), out, rows, None, S(T, HQ, HKV, D, n, past), 3,
+                                ops.Qwen35AttentionLaunchPolicy(1, 0, 0))
+    torch.cuda.synchronize()
+    p = torch.softmax(rows[0, :past, 0, 0].double(), 0)
+    want = 0.5 * (p * rows[1, :past, 0, 0].double()).sum().item()  # the new keys' weight is e^-1000
+    # bf16 rounding of the output; a score of 1000 carries 6e-5 in f32, which moves each weight by as much
+    assert abs(out[0, 0, 0].item() - want) <= (2.0 ** -8 + 1e-3) * want
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_f32_cache_prefill_infinite_values(gpu, value):
+    # An infinite V row reaches exactly the tokens that see it, on past and new rows, as in a scalar sum.
+    T, past = 20, 21
+    rows_hit = [5, past + 7]
+
+    def edit(rows):
+        for r in rows_hit:
+            rows[1, r, 1, 3] = value
+
+    out, p, v, gate, hidden, _ = f32_cache(T, past, 0, seed=3, edit=edit)
+    got = from_dev(out)
+    finite = torch.where(torch.isfinite(v), v, torch.zeros_like(v))
+    want = (torch.matmul(p, finite).permute(1, 0, 2) * torch.sigmoid(gate)).cpu().numpy()
+    # every token sees row 5; column (head 4..7, dim 3) is infinite (NaN for NaN), all others as without it
+    hit = np.zeros_like(want, bool)
+    hit[:, 4:8, 3] = True
+    assert np.all(np.abs(got - want)[~hit] <= 2.0 ** -8 * np.abs(want[~hit]) * 1.001 + 2e-5)
+    assert np.isnan(got[hit]).all() if np.isnan(value) else (got[hit] == value).all()
+
+    def edit_new(rows):
+        rows[1, past + 7, 1, 3] = value
+
+    out, p, v, gate, hidden, _ = f32_cache(T, past, 0, seed=3, edit=edit_new)
+    got = from_dev(out)
+    assert np.isfinite(got[:7]).all() and not np.isfinite(got[7:, 4:8, 3]).any()
+    mask = np.ones_like(got, bool)
+    mask[7:, 4:8, 3] = False
+    assert np.isfinite(got[mask]).all()
