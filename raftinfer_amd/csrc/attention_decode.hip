@@ -114,96 +114,6 @@ __device__ __forceinline__ std::size_t read_position(const std::uint32_t *device
   return device_position == nullptr ? host_position : static_cast<std::size_t>(*device_position);
 }
 
-// Writes one token's K and V (4 x 256 each) at the position, RNE-cast to
-// the cache dtype.  Grid: 4 x 256.
-template <typename ActT, typename CacheT>
-__global__ __launch_bounds__(256) void append_decode_kernel(
-    const ActT *__restrict__ key, const ActT *__restrict__ value, CacheT *__restrict__ cache,
-    std::size_t max_ctx, std::size_t host_position, bool head_major,
-    const std::uint32_t *device_position) {
-  const std::size_t position = read_position(device_position, host_position);
-  if (position >= max_ctx) return;
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  const int kvh = e >> 8;
-  const int d = e & 255;
-  const std::size_t idx = cache_row(head_major, position, kvh, max_ctx) + d;
-  const std::size_t plane = max_ctx * kKvHeads * kHeadDim;
-  Elem<CacheT>::store(cache, idx, Elem<ActT>::load(key, e));
-  Elem<CacheT>::store(cache, plane + idx, Elem<ActT>::load(value, e));
-}
-
-// Zero-workspace single-block decode: one workgroup per group of NH query
-// heads scans the whole context and writes the gated output.  Exits when the
-// plan's split threshold is reached (mirrors the device-side early exit of
-// cpp/kernels/qwen35_online_attention.cu:427-430).
-template <typename ActT, typename CacheT, int NH, int WAVES, int U>
-__global__ __launch_bounds__(WAVES * 64) void decode_single_block_kernel(
-    const ActT *__restrict__ query, const ActT *__restrict__ gate, ActT *__restrict__ output,
-    const CacheT *__restrict__ cache, std::size_t max_ctx, std::size_t host_position,
-    bool head_major, const std::uint32_t *device_position, std::size_t threshold) {
-  __shared__ ScanShared<NH, WAVES> sh;
-  const std::size_t position = read_position(device_position, host_position);
-  if (position >= max_ctx) return;
-  const std::size_t ctx = position + 1;
-  if (threshold != 0 && ctx >= threshold) return;
-  const std::size_t first_head = static_cast<std::size_t>(blockIdx.x) * NH;
-  const std::size_t kv_head = first_head / kGroup;
-  const CacheT *k_plane = cache;
-  const CacheT *v_plane = cache + max_ctx * kKvHeads * kHeadDim;
-  scan_range<ActT, CacheT, NH, WAVES, U>(query, first_head, k_plane, v_plane, head_major, max_ctx,
-                                         kv_head, 0, ctx, sh);
-  __syncthreads();
-  for (int o = threadIdx.x; o < NH * kHeadDim; o += WAVES * 64) {
-    const int h = o / kHeadDim, d = o % kHeadDim;
-    float mm, l, a;
-    combine_waves(sh, h, d, mm, l, a);
-    const std::size_t out_idx = (first_head + h) * kHeadDim + d;
-    const float gv = Elem<ActT>::load(gate, out_idx);
-    Elem<ActT>::store(output, out_idx, (a / l) * sigmoid_gate(gv));
-  }
-}
-
-// Split-K partition: workgroup (head group, partition p) scans tokens
-// [p*P, min(ctx, (p+1)*P)) and writes fp32 (max, sum, value[256]) per query
-// head at index qh*max_partitions + p, the reference workspace bookkeeping
-// (cpp/kernels/qwen35_online_attention.cu:602-691).
-template <typename ActT, typename CacheT, int NH, int WAVES, int U>
-__global__ __launch_bounds__(WAVES * 64) void decode_partition_kernel(
-    const ActT *__restrict__ query, const CacheT *__restrict__ cache, float *__restrict__ pmax,
-    float *__restrict__ psum, float *__restrict__ pval, std::size_t max_ctx,
-    std::size_t host_position, bool head_major, std::size_t capacity,
-    std::size_t max_partitions, std::size_t partition_tokens, std::size_t threshold,
-    const std::uint32_t *device_position) {
-  __shared__ ScanShared<NH, WAVES> sh;
-  const std::size_t position = read_position(device_position, host_position);
-  if (position >= max_ctx) return;
-  const std::size_t ctx = position + 1;
-  if (ctx < threshold) return;
-  const std::size_t unit = blockIdx.x / capacity;
-  const std::size_t partition = blockIdx.x % capacity;
-  const std::size_t begin = partition * partition_tokens;
-  if (begin >= ctx) return;
-  const std::size_t end = ctx < begin + partition_tokens ? ctx : begin + partition_tokens;
-  const std::size_t first_head = unit * NH;
-  const std::size_t kv_head = first_head / kGroup;
-  const CacheT *k_plane = cache;
-  const CacheT *v_plane = cache + max_ctx * kKvHeads * kHeadDim;
-  scan_range<ActT, CacheT, NH, WAVES, U>(query, first_head, k_plane, v_plane, head_major, max_ctx,
-                                         kv_head, begin, end, sh);
-  __syncthreads();
-  for (int o = threadIdx.x; o < NH * kHeadDim; o += WAVES * 64) {
-    const int h = o / kHeadDim, d = o % kHeadDim;
-    float mm, l, a;
-    combine_waves(sh, h, d, mm, l, a);
-    const std::size_t idx = (first_head + h) * max_partitions + partition;
-    if (d == 0) {
-      pmax[idx] = mm * kLn2;
-      psum[idx] = l;
-    }
-    pval[idx * kHeadDim + d] = a;
-  }
-}
-
 // Log-sum-exp merge over the active partitions of one query head plus the
 // sigmoid gate (cpp/kernels/qwen35_online_attention.cu:693-756).  The value
 // loads of a chunk do not wait for its max / sum, so they are all independent.
@@ -704,6 +614,107 @@ __global__ __launch_bounds__(WAVES * 64) void decode_dynamic_mfma_kernel(
                                       max_partitions, partition_tokens, f, psh, fq);
 }
 
+// ---- f32 activations or f32 caches (scan_slice).  The same split of the work
+// as the bf16 kernels: a workgroup per (KV head, partition, dims slice), the
+// slices of a partition on one XCD, each computing the scores of all its keys and
+// reading its own part of V.  With the whole 256 dims in one workgroup a context
+// of 3000 tokens had 48 workgroups, and a step was four launches (append, early
+// exit of the single-block kernel, partitions, merge): 26.5 us on an f32
+// token-major cache, 15 of them the partitions.  Sliced, with the append and the
+// choice of path inside, it is two launches and 15.8 us (partitions 11.4: 320 KiB of
+// plain loads per CU at about 33 B/clk, then their FMAs).
+constexpr int kScanWaves = 8;
+constexpr int scan_unroll(int ds) { return ds == 1 ? 2 : 4; } // tokens per row-group and step (registers)
+
+template <typename ActT, typename CacheT>
+__device__ __forceinline__ void scan_single_body(unsigned block, const ScanArgs<ActT, CacheT> &a,
+                                                 const ActT *__restrict__ gate, ActT *__restrict__ output,
+                                                 std::size_t position, ScanShared<kSingleDs, kScanWaves> &sh) {
+  constexpr int DS = kSingleDs, kDims = kHeadDim / DS;
+  std::size_t kv_head;
+  int dq;
+  xcd_unit<DS>(block, kv_head, dq);
+  if (kv_head >= kKvHeads) return;
+  const int o = threadIdx.x, h = o / kDims, d = o % kDims; // the first 4 x 16 threads finish an output
+  const std::size_t idx = (kv_head * kGroup + h) * kHeadDim + dq * kDims + d;
+  const bool finisher = o < kGroup * kDims;
+  const float gv = finisher ? Elem<ActT>::load(gate, idx) : 0.f;
+  scan_slice<ActT, CacheT, DS, kScanWaves, scan_unroll(DS)>(a, kv_head, dq, 0, position + 1, position, sh);
+  __syncthreads();
+  if (dq == 0) append_rows(a, kv_head, position);
+  if (!finisher) return;
+  float mm, l, acc;
+  combine_waves(sh, h, d, mm, l, acc);
+  Elem<ActT>::store(output, idx, (acc / l) * sigmoid_gate(gv));
+}
+
+template <typename ActT, typename CacheT, int DS>
+__device__ __forceinline__ void scan_split_body(unsigned block, const ScanArgs<ActT, CacheT> &a,
+                                                float *__restrict__ pmax, float *__restrict__ psum,
+                                                float *__restrict__ pval, std::size_t position,
+                                                std::size_t capacity, std::size_t max_partitions,
+                                                std::size_t partition_tokens, ScanShared<DS, kScanWaves> &sh) {
+  constexpr int kDims = kHeadDim / DS;
+  const std::size_t ctx = position + 1;
+  std::size_t unit;
+  int dq;
+  xcd_unit<DS>(block, unit, dq);
+  if (unit >= kKvHeads * capacity) return;
+  const std::size_t kv_head = DS == 1 ? unit % kKvHeads : unit / capacity;
+  const std::size_t partition = DS == 1 ? unit / kKvHeads : unit % capacity;
+  const std::size_t begin = partition * partition_tokens;
+  if (begin >= ctx) return;
+  const std::size_t end = ctx < begin + partition_tokens ? ctx : begin + partition_tokens;
+  scan_slice<ActT, CacheT, DS, kScanWaves, scan_unroll(DS)>(a, kv_head, dq, begin, end, position, sh);
+  __syncthreads();
+  // the append, also of a position past the plan's capacity (see split_body)
+  const bool owns_position = position >= begin && position < end;
+  const bool past_capacity = partition + 1 == capacity && position >= begin + partition_tokens;
+  if (dq == 0 && (owns_position || past_capacity)) append_rows(a, kv_head, position);
+  for (int o = threadIdx.x; o < kGroup * kDims; o += kScanWaves * 64) {
+    const int h = o / kDims, d = o % kDims;
+    float mm, l, acc;
+    combine_waves(sh, h, d, mm, l, acc);
+    const std::size_t idx = (kv_head * kGroup + h) * max_partitions + partition;
+    if (dq == 0 && d == 0) {
+      pmax[idx] = mm * kLn2;
+      psum[idx] = l;
+    }
+    pval[idx * kHeadDim + dq * kDims + d] = acc;
+  }
+}
+
+template <typename ActT, typename CacheT>
+__global__ __launch_bounds__(kScanWaves * 64) void decode_scan_single_kernel(
+    ScanArgs<ActT, CacheT> a, const ActT *__restrict__ gate, ActT *__restrict__ output, std::size_t host_position,
+    const std::uint32_t *device_position) {
+  __shared__ ScanShared<kSingleDs, kScanWaves> sh;
+  const std::size_t position = read_position(device_position, host_position);
+  if (position >= a.max_ctx) return;
+  scan_single_body(blockIdx.x, a, gate, output, position, sh);
+}
+
+// One launch for both sides of the split threshold (the single-block work in
+// the first blocks below it), so that a device position selects on the device.
+template <typename ActT, typename CacheT, int DS>
+__global__ __launch_bounds__(kScanWaves * 64) void decode_scan_kernel(
+    ScanArgs<ActT, CacheT> a, const ActT *__restrict__ gate, ActT *__restrict__ output, float *__restrict__ pmax,
+    float *__restrict__ psum, float *__restrict__ pval, std::size_t host_position,
+    const std::uint32_t *device_position, std::size_t capacity, std::size_t max_partitions,
+    std::size_t partition_tokens, std::size_t threshold, bool partition_only) {
+  __shared__ union Shared {
+    ScanShared<kSingleDs, kScanWaves> single;
+    ScanShared<DS, kScanWaves> split;
+  } sh;
+  const std::size_t position = read_position(device_position, host_position);
+  if (position >= a.max_ctx) return;
+  if (position + 1 >= threshold)
+    scan_split_body<ActT, CacheT, DS>(blockIdx.x, a, pmax, psum, pval, position, capacity, max_partitions,
+                                      partition_tokens, sh.split);
+  else if (!partition_only)
+    scan_single_body(blockIdx.x, a, gate, output, position, sh.single);
+}
+
 // ------------------------------------------------------------ launchers
 
 // Plans of at most 16 partitions (ctx 4096 at P=256) use the 64-workgroup
@@ -845,9 +856,6 @@ void launch_decode_mfma(const DecodeMfmaArgs &args, const bf16_bits *g, std::siz
   check_launch<Err>("qwen35_online_attention_decode_split_k_merge");
 }
 
-constexpr int kSingleHeads = 1, kSingleWaves = 16, kSingleUnroll = 2;
-constexpr int kPartHeads = 4, kPartWaves = 8, kPartUnroll = 2;
-
 template <typename ActT, typename CacheT>
 void launch_decode(const void *query, const void *key, const void *value, const void *gate,
                    void *output, void *kv_cache, void *workspace, Qwen35AttentionShape shape,
@@ -865,54 +873,50 @@ void launch_decode(const void *query, const void *key, const void *value, const 
                               shape.max_context_tokens, head_major};
     launch_decode_mfma<false>(args, g, kHeadDim, out, workspace, shape, plan, ws, device_position,
                               stream, partition_only, FusedNormRope{});
+  } else {
+  const bool single = plan.resolved_mode == Qwen35DecodeAttentionMode::single_block;
+  if (partition_only) require<Err>(plan.partition_tokens != 0, "partition-only decode needs a split-K plan");
+  const ScanArgs<ActT, CacheT> args{q, static_cast<const ActT *>(key), static_cast<const ActT *>(value), cache,
+                                    shape.max_context_tokens, head_major};
+  const unsigned single_grid = xcd_grid<kSingleDs>(kKvHeads);
+  const std::size_t host_ctx = shape.past_tokens + 1;
+  if (single || (device_position == nullptr && !partition_only && host_ctx < plan.split_k_threshold_tokens)) {
+    decode_scan_single_kernel<ActT, CacheT><<<single_grid, kScanWaves * 64, 0, stream>>>(
+        args, g, out, shape.past_tokens, device_position);
+    check_launch<Err>("qwen35_online_attention_decode_gfx950_hd256");
     return;
   }
-  if (partition_only) {
-    require<Err>(plan.partition_tokens != 0, "partition-only decode needs a split-K plan");
-  } else {
-  append_decode_kernel<ActT, CacheT><<<4, 256, 0, stream>>>(
-      static_cast<const ActT *>(key), static_cast<const ActT *>(value), cache,
-      shape.max_context_tokens, shape.past_tokens, head_major, device_position);
-  check_launch<Err>("qwen35_online_attention_decode_append_cache");
-  }
-
-  // With a host position the path is known here, so kernels that would only
-  // early-exit are not enqueued.  With a device position every kernel of the
-  // plan is enqueued and selects itself on-device (graph-capture safe).
-  const std::size_t host_ctx = shape.past_tokens + 1;
-  const bool dynamic = device_position != nullptr;
-  const bool single = plan.resolved_mode == Qwen35DecodeAttentionMode::single_block;
-  if (!partition_only && (dynamic || single || host_ctx < plan.split_k_threshold_tokens)) {
-    decode_single_block_kernel<ActT, CacheT, kSingleHeads, kSingleWaves, kSingleUnroll>
-        <<<kQueryHeads / kSingleHeads, kSingleWaves * 64, 0, stream>>>(
-            q, g, out, cache, shape.max_context_tokens, shape.past_tokens, head_major,
-            device_position, plan.split_k_threshold_tokens);
-    check_launch<Err>("qwen35_online_attention_decode_gfx950_hd256");
-  }
-  if (single) return;
-  if (!dynamic && host_ctx < plan.split_k_threshold_tokens) return;
-
   const std::size_t max_partitions = ceil_div(shape.max_context_tokens, plan.partition_tokens,
                                               "online decode maximum partition capacity overflow");
-  const std::size_t units = kQueryHeads / kPartHeads;
-  const int grid = grid_dim(checked_mul<Err>(units, plan.active_partition_capacity,
-                                             "online decode partition grid dimension overflow"),
-                            "online decode partition grid dimension overflow");
+  const std::size_t units = checked_mul<Err>(kKvHeads, plan.active_partition_capacity,
+                                             "online decode partition grid dimension overflow");
+  (void)grid_dim(checked_mul<Err>(units + 8, kSplitDs, "online decode partition grid dimension overflow"),
+                 "online decode partition grid dimension overflow");
   auto *bytes = static_cast<std::byte *>(workspace);
   auto *pmax = reinterpret_cast<float *>(bytes + ws.max_offset_bytes);
   auto *psum = reinterpret_cast<float *>(bytes + ws.sum_offset_bytes);
   auto *pval = reinterpret_cast<float *>(bytes + ws.value_offset_bytes);
-  decode_partition_kernel<ActT, CacheT, kPartHeads, kPartWaves, kPartUnroll>
-      <<<grid, kPartWaves * 64, 0, stream>>>(
-          q, cache, pmax, psum, pval, shape.max_context_tokens, shape.past_tokens, head_major,
-          plan.active_partition_capacity, max_partitions, plan.partition_tokens,
-          plan.split_k_threshold_tokens, device_position);
+  // As the bf16 kernels: slice the dims only while the partitions alone leave
+  // the 256 CUs idle.
+  auto go = [&](auto kernel, unsigned split_grid) {
+    kernel<<<split_grid > single_grid ? split_grid : single_grid, kScanWaves * 64, 0, stream>>>(
+        args, g, out, pmax, psum, pval, shape.past_tokens, device_position, plan.active_partition_capacity,
+        max_partitions, plan.partition_tokens, plan.split_k_threshold_tokens, partition_only);
+  };
+  if (units >= 192)
+    go(decode_scan_kernel<ActT, CacheT, 1>, xcd_grid<1>(units));
+  else if (units >= 96)
+    go(decode_scan_kernel<ActT, CacheT, 2>, xcd_grid<2>(units));
+  else
+    go(decode_scan_kernel<ActT, CacheT, kSplitDs>, xcd_grid<kSplitDs>(units));
   check_launch<Err>(plan.partition_tokens == 256
                         ? "qwen35_online_attention_decode_split_k_256_partition"
                         : "qwen35_online_attention_decode_split_k_512_partition");
+  if (partition_only) return;
   launch_merge<ActT>(g, kHeadDim, out, pmax, psum, pval, shape, plan, max_partitions, device_position,
                      stream);
   check_launch<Err>("qwen35_online_attention_decode_split_k_merge");
+  }
 }
 
 void require_aligned16(const void *p, const char *message) {
@@ -1216,18 +1220,17 @@ namespace {
 
 constexpr std::size_t kBatchedPartition = 256;
 
-// Workgroup (sequence, head group, partition).  Sequences whose context is at
+// Workgroup (sequence, KV head, partition).  Sequences whose context is at
 // most single_max run single-block in partition 0 and write the gated output;
 // longer ones write partials for the merge.
-template <typename ActT, int NH, int WAVES, int U>
+template <typename ActT, int WAVES, int U>
 __global__ __launch_bounds__(WAVES * 64) void batched_partition_kernel(
     const ActT *__restrict__ query, const ActT *__restrict__ key, const ActT *__restrict__ value,
-    const ActT *__restrict__ gate, ActT *__restrict__ output, const std::byte *cache_base,
+    const ActT *__restrict__ gate, ActT *__restrict__ output, std::byte *cache_base,
     std::size_t cache_stride, std::size_t max_ctx, const std::uint32_t *__restrict__ lengths,
     std::size_t max_partitions, std::size_t single_max, float *__restrict__ pmax,
     float *__restrict__ psum, float *__restrict__ pval) {
-  __shared__ ScanShared<NH, WAVES> sh;
-  constexpr std::size_t units = kQueryHeads / NH;
+  __shared__ ScanShared<1, WAVES> sh;
   const std::size_t seq = blockIdx.y;
   const std::size_t unit = blockIdx.x / max_partitions;
   const std::size_t partition = blockIdx.x % max_partitions;
@@ -1237,54 +1240,29 @@ __global__ __launch_bounds__(WAVES * 64) void batched_partition_kernel(
   const std::size_t begin = partition * kBatchedPartition;
   if (single ? partition != 0 : begin >= ctx) return;
   const std::size_t end = single ? ctx : (ctx < begin + kBatchedPartition ? ctx : begin + kBatchedPartition);
-  const auto *cache = reinterpret_cast<const bf16_bits *>(cache_base + seq * cache_stride);
-  const std::size_t first_head = unit * NH;
-  const std::size_t kv_head = first_head / kGroup;
-  const bf16_bits *k_plane = cache;
-  const bf16_bits *v_plane = cache + max_ctx * kKvHeads * kHeadDim;
-  const ActT *q = query + seq * kQueryHeads * kHeadDim;
-  scan_range<ActT, bf16_bits, NH, WAVES, U>(q, first_head, k_plane, v_plane, true, max_ctx,
-                                            kv_head, begin, end, sh);
+  const ScanArgs<ActT, bf16_bits> a{query + seq * kQueryHeads * kHeadDim, key + seq * kKvHeads * kHeadDim,
+                                    value + seq * kKvHeads * kHeadDim,
+                                    reinterpret_cast<bf16_bits *>(cache_base + seq * cache_stride), max_ctx, true};
+  scan_slice<ActT, bf16_bits, 1, WAVES, U>(a, unit, 0, begin, end, ctx - 1, sh);
   __syncthreads();
-  for (int o = threadIdx.x; o < NH * kHeadDim; o += WAVES * 64) {
+  if (ctx - 1 >= begin && ctx - 1 < end) append_rows(a, unit, ctx - 1);
+  for (int o = threadIdx.x; o < kGroup * kHeadDim; o += WAVES * 64) {
     const int h = o / kHeadDim, d = o % kHeadDim;
-    float mm, l, a;
-    combine_waves(sh, h, d, mm, l, a);
-    const std::size_t head = first_head + h;
+    float mm, l, acc;
+    combine_waves(sh, h, d, mm, l, acc);
+    const std::size_t head = unit * kGroup + h;
     if (single) {
       const std::size_t out_idx = (seq * kQueryHeads + head) * kHeadDim + d;
-      Elem<ActT>::store(output, out_idx, (a / l) * sigmoid_gate(Elem<ActT>::load(gate, out_idx)));
+      Elem<ActT>::store(output, out_idx, (acc / l) * sigmoid_gate(Elem<ActT>::load(gate, out_idx)));
     } else {
       const std::size_t idx = (seq * kQueryHeads + head) * max_partitions + partition;
       if (d == 0) {
         pmax[idx] = mm * kLn2;
         psum[idx] = l;
       }
-      pval[idx * kHeadDim + d] = a;
+      pval[idx * kHeadDim + d] = acc;
     }
   }
-  (void)units;
-  (void)key;
-  (void)value;
-}
-
-template <typename ActT>
-__global__ __launch_bounds__(256) void batched_append_kernel(const ActT *__restrict__ key,
-                                                             const ActT *__restrict__ value,
-                                                             std::byte *cache_base,
-                                                             std::size_t cache_stride,
-                                                             std::size_t max_ctx,
-                                                             const std::uint32_t *lengths) {
-  const std::size_t seq = blockIdx.y;
-  const std::size_t ctx = lengths[seq];
-  if (ctx == 0 || ctx > max_ctx) return;
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  auto *cache = reinterpret_cast<bf16_bits *>(cache_base + seq * cache_stride);
-  const std::size_t idx = cache_row(true, ctx - 1, e >> 8, max_ctx) + (e & 255);
-  const std::size_t plane = max_ctx * kKvHeads * kHeadDim;
-  const std::size_t src = seq * kKvHeads * kHeadDim + e;
-  cache[idx] = f32_to_bf16(Elem<ActT>::load(key, src));
-  cache[plane + idx] = f32_to_bf16(Elem<ActT>::load(value, src));
 }
 
 // Workgroup = (sequence, head), kBatchedMergeWaves waves, so a 32768-token
@@ -1424,12 +1402,9 @@ void launch_batched(const void *query, const void *key, const void *value, const
     check_launch<Err>("qwen35_batched_decode_merge");
     return;
   }
-  batched_append_kernel<ActT><<<dim3(4, seqs), 256, 0, stream>>>(
-      k, v, base, shape.cache_stride_bytes, shape.max_context_tokens, lengths);
-  check_launch<Err>("qwen35_batched_decode_append_cache");
-  constexpr int NH = 4, WAVES = 8, U = 2;
-  const unsigned int gx = static_cast<unsigned int>((kQueryHeads / NH) * max_partitions);
-  batched_partition_kernel<ActT, NH, WAVES, U><<<dim3(gx, seqs), WAVES * 64, 0, stream>>>(
+  constexpr int WAVES = 8, U = 2;
+  const unsigned int gx = static_cast<unsigned int>(kKvHeads * max_partitions);
+  batched_partition_kernel<ActT, WAVES, U><<<dim3(gx, seqs), WAVES * 64, 0, stream>>>(
       q, k, v, g, out, base, shape.cache_stride_bytes, shape.max_context_tokens, lengths,
       max_partitions, shape.single_block_max_tokens, pmax, psum, pval);
   check_launch<Err>("qwen35_batched_decode_partition");

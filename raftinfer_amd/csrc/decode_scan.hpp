@@ -1,12 +1,11 @@
-// Device core shared by the single-block, split-K and batched decode kernels:
-// one workgroup scans a token range of one KV head for NH query heads of its
-// GQA group, keeping an online-softmax state per head.
+// Device core of the decode kernels for f32 activations or f32 caches (the
+// bf16 / bf16 kernels have theirs in decode_mfma.hpp): one workgroup scans a
+// token range of one KV head for the four query heads of its GQA group and one
+// slice of the output dims, keeping an online-softmax state per head.
 //
-// Lane layout (wave64 = 4 row-groups of 16 lanes): row-group g takes one
-// token per step, lane r of the group owns dims [8r, 8r+8) and
-// [128+8r, 128+8r+8) of the 256-wide head, so one 16-byte load per lane per
-// half-row gives each 16-lane group a contiguous 256-byte half of a K or V
-// row (full 128-byte lines, coalesced).  q.k partial dots reduce inside the
+// Lane layout (wave64 = 4 row-groups of 16 lanes): row-group g takes one token
+// per step, and a row is read in 16-byte pieces, 16 lanes on one contiguous
+// 256-byte stretch (whole 128-byte lines).  q.k partial dots reduce inside the
 // 16-lane row with four DPP steps; the softmax runs in the exp2 domain with
 // log2(e)/sqrt(D) folded into q.
 #pragma once
@@ -22,36 +21,6 @@ constexpr int kGroup = kQueryHeads / kKvHeads;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
-template <typename T> struct Chunk8;
-template <> struct Chunk8<bf16_bits> {
-  u32x4 w;
-  __device__ __forceinline__ void load(const bf16_bits *p) {
-    w = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
-  }
-  __device__ __forceinline__ void zero() { w = u32x4{0u, 0u, 0u, 0u}; }
-  __device__ __forceinline__ float get(int i) const {
-    const std::uint32_t x = w[i >> 1];
-    return (i & 1) ? bf16_hi(x) : bf16_lo(x);
-  }
-};
-template <> struct Chunk8<float> {
-  float4 a, b;
-  __device__ __forceinline__ void load(const float *p) {
-    a = reinterpret_cast<const float4 *>(p)[0];
-    b = reinterpret_cast<const float4 *>(p)[1];
-  }
-  __device__ __forceinline__ void zero() {
-    a = make_float4(0.f, 0.f, 0.f, 0.f);
-    b = a;
-  }
-  __device__ __forceinline__ float get(int i) const {
-    switch (i) {
-    case 0: return a.x; case 1: return a.y; case 2: return a.z; case 3: return a.w;
-    case 4: return b.x; case 5: return b.y; case 6: return b.z; default: return b.w;
-    }
-  }
-};
-
 // Element index of (token, kv_head, dim 0) in one cache plane
 // (cpp/kernels/qwen35_online_attention.cu:240-252).
 __device__ __forceinline__ std::size_t cache_row(bool head_major, std::size_t token,
@@ -60,110 +29,163 @@ __device__ __forceinline__ std::size_t cache_row(bool head_major, std::size_t to
                     : (token * kKvHeads + kv_head) * kHeadDim;
 }
 
-// Per-head combined state after a workgroup scan, staged in LDS.
-template <int NH, int WAVES> struct ScanShared {
-  float m[WAVES][NH];
-  float l[WAVES][NH];
-  float acc[WAVES][NH][kHeadDim];
+// W contiguous cache elements as loaded (kOnce: read by one workgroup only, so
+// streamed past the caches).
+template <typename T, int W, bool kOnce> struct Piece {
+  static_assert(W * sizeof(T) <= 16);
+  typedef T vec __attribute__((ext_vector_type(W == 1 ? 2 : W)));
+  using Raw = std::conditional_t<W == 1, T, vec>;
+  Raw raw;
+  __device__ __forceinline__ void load(const T *p) {
+    const auto *v = reinterpret_cast<const Raw *>(p);
+    if constexpr (kOnce) raw = __builtin_nontemporal_load(v); else raw = *v;
+  }
+  __device__ __forceinline__ void set(int i, T x) {
+    if constexpr (W == 1) raw = x; else raw[i] = x;
+  }
+  __device__ __forceinline__ float get(int i) const {
+    T x;
+    if constexpr (W == 1) x = raw; else x = raw[i];
+    return Elem<T>::load(&x, 0);
+  }
 };
 
-// Scans tokens [begin, end) of kv_head for query heads first_head..+NH and
-// leaves the per-wave states in `sh`.  Every wave returns after writing its
-// slot; the caller synchronizes.
-template <typename ActT, typename CacheT, int NH, int WAVES, int U>
-__device__ __forceinline__ void scan_range(const ActT *__restrict__ query, std::size_t first_head,
-                                           const CacheT *__restrict__ k_plane,
-                                           const CacheT *__restrict__ v_plane, bool head_major,
-                                           std::size_t max_ctx, std::size_t kv_head,
-                                           std::size_t begin, std::size_t end,
-                                           ScanShared<NH, WAVES> &sh) {
+// What the scan reads: query [16][256], the new token's key / value rows
+// [4][256] (its cache rows are not read) and the cache planes.
+template <typename ActT, typename CacheT> struct ScanArgs {
+  const ActT *query, *key_new, *value_new;
+  CacheT *cache;
+  std::size_t max_ctx;
+  bool head_major;
+};
+
+// Per-head combined state after a workgroup scan, staged in LDS.
+template <int DS, int WAVES> struct ScanShared {
+  float m[WAVES][kGroup];
+  float l[WAVES][kGroup];
+  float acc[WAVES][kGroup][kHeadDim / DS];
+};
+
+// Scans tokens [begin, end) of kv_head, dims slice dq of 256 / DS for the
+// output, and leaves the per-wave states in `sh`.  The row of position `pos` (if
+// in range) comes from key_new / value_new, as the cache stores it.  U tokens per
+// row-group and step.  Every wave returns after writing its slot; the caller
+// synchronizes.
+template <typename ActT, typename CacheT, int DS, int WAVES, int U>
+__device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std::size_t kv_head, int dq,
+                                           std::size_t begin, std::size_t end, std::size_t pos,
+                                           ScanShared<DS, WAVES> &sh) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int g = lane >> 4;
   const int r = lane & 15;
   const float qscale = kLog2e / 16.0f; // log2(e) / sqrt(256)
+  constexpr int kDims = kHeadDim / DS, kPerLane = kDims / 16; // output dims of the slice, of a lane
+  constexpr int KW = 16 / sizeof(CacheT), KP = 16 / KW;       // K piece width, pieces per lane
+  constexpr int VW = kPerLane < KW ? kPerLane : KW, VP = kPerLane / VW;
+  // Element of piece p of a lane: 16 KW p + KW r (K), 16 VW p + VW r of the slice (V).
+  const CacheT *k_plane = a.cache + cache_row(a.head_major, 0, kv_head, a.max_ctx);
+  const CacheT *v_plane = k_plane + a.max_ctx * kKvHeads * kHeadDim + dq * kDims;
+  const std::size_t token_stride = a.head_major ? kHeadDim : kKvHeads * kHeadDim;
 
-  float q[NH][16];
+  float q[kGroup][16];
 #pragma unroll
-  for (int h = 0; h < NH; ++h) {
-    const ActT *qh = query + (first_head + h) * kHeadDim;
+  for (int h = 0; h < kGroup; ++h) {
+    const ActT *qh = a.query + (kv_head * kGroup + h) * kHeadDim;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      q[h][i] = Elem<ActT>::load(qh, 8 * r + i) * qscale;
-      q[h][8 + i] = Elem<ActT>::load(qh, 128 + 8 * r + i) * qscale;
-    }
+    for (int i = 0; i < 16; ++i) q[h][i] = Elem<ActT>::load(qh, 16 * KW * (i / KW) + KW * r + i % KW) * qscale;
   }
 
-  float m[NH], l[NH], acc[NH][16];
+  float m[kGroup], l[kGroup], acc[kGroup][kPerLane];
 #pragma unroll
-  for (int h = 0; h < NH; ++h) {
+  for (int h = 0; h < kGroup; ++h) {
     m[h] = -INFINITY;
     l[h] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[h][i] = 0.f;
+    for (int i = 0; i < kPerLane; ++i) acc[h][i] = 0.f;
   }
 
   constexpr int kTile = 4 * U; // tokens per wave step
   for (std::size_t tile = begin + static_cast<std::size_t>(wave) * kTile; tile < end;
        tile += static_cast<std::size_t>(WAVES) * kTile) {
-    Chunk8<CacheT> ka[U], kb[U], va[U], vb[U];
-    bool valid[U];
+    Piece<CacheT, KW, DS == 1> k[U][KP];
+    Piece<CacheT, VW, true> v[U][VP];
+    const bool whole = tile + kTile <= end; // (uniform)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
+      // tokens past the range re-read its last row (masked below)
       const std::size_t tok = tile + 4 * u + g;
-      valid[u] = tok < end;
-      if (valid[u]) {
-        const std::size_t row = cache_row(head_major, tok, kv_head, max_ctx) + 8 * r;
-        ka[u].load(k_plane + row);
-        kb[u].load(k_plane + row + 128);
-        va[u].load(v_plane + row);
-        vb[u].load(v_plane + row + 128);
-      } else {
-        ka[u].zero();
-        kb[u].zero();
-        va[u].zero();
-        vb[u].zero();
+      const std::size_t row = (tok < end ? tok : end - 1) * token_stride;
+#pragma unroll
+      for (int p = 0; p < KP; ++p) k[u][p].load(k_plane + row + 16 * KW * p + KW * r);
+#pragma unroll
+      for (int p = 0; p < VP; ++p) v[u][p].load(v_plane + row + 16 * VW * p + VW * r);
+    }
+    if (pos >= tile && pos < tile + kTile) { // (uniform) this step holds the new token
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (tile + 4 * u + g != pos) continue;
+        const ActT *kn = a.key_new + kv_head * kHeadDim, *vn = a.value_new + kv_head * kHeadDim + dq * kDims;
+        CacheT x;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          Elem<CacheT>::store(&x, 0, Elem<ActT>::load(kn, 16 * KW * (i / KW) + KW * r + i % KW));
+          k[u][i / KW].set(i % KW, x);
+        }
+#pragma unroll
+        for (int i = 0; i < kPerLane; ++i) {
+          Elem<CacheT>::store(&x, 0, Elem<ActT>::load(vn, 16 * VW * (i / VW) + VW * r + i % VW));
+          v[u][i / VW].set(i % VW, x);
+        }
       }
     }
-    float s[NH][U];
+    float s[kGroup][U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
-      for (int h = 0; h < NH; ++h) {
+      for (int h = 0; h < kGroup; ++h) {
         float d0 = 0.f, d1 = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-          d0 = fmaf(q[h][i], ka[u].get(i), d0);
-          d1 = fmaf(q[h][8 + i], kb[u].get(i), d1);
+          d0 = fmaf(q[h][i], k[u][i / KW].get(i % KW), d0);
+          d1 = fmaf(q[h][8 + i], k[u][(8 + i) / KW].get((8 + i) % KW), d1);
         }
         s[h][u] = row16_sum(d0 + d1);
       }
     }
+    if (!whole) {
+      // no weight, and no value either: the row read in its place may be the
+      // new token's, which the cache does not hold yet
 #pragma unroll
-    for (int h = 0; h < NH; ++h) {
+      for (int u = 0; u < U; ++u) {
+        if (tile + 4 * u + g < end) continue;
+#pragma unroll
+        for (int h = 0; h < kGroup; ++h) s[h][u] = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < kPerLane; ++i) v[u][i / VW].set(i % VW, CacheT{});
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < kGroup; ++h) {
       float mt = m[h];
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (valid[u]) mt = fmaxf(mt, s[h][u]);
-      const float so = m[h] == -INFINITY ? 0.f : exp2f(m[h] - mt);
+      for (int u = 0; u < U; ++u) mt = fmaxf(mt, s[h][u]);
+      const float ref = mt == -INFINITY ? 0.f : mt; // a row-group may have seen no token yet
+      const float so = __builtin_amdgcn_exp2f(m[h] - ref);
       float p[U];
       float psum = 0.f;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        p[u] = valid[u] ? exp2f(s[h][u] - mt) : 0.f;
+        p[u] = __builtin_amdgcn_exp2f(s[h][u] - ref);
         psum += p[u];
       }
       l[h] = l[h] * so + psum;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float a0 = acc[h][i] * so, a1 = acc[h][8 + i] * so;
+      for (int i = 0; i < kPerLane; ++i) {
+        float x = acc[h][i] * so;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          a0 = fmaf(p[u], va[u].get(i), a0);
-          a1 = fmaf(p[u], vb[u].get(i), a1);
-        }
-        acc[h][i] = a0;
-        acc[h][8 + i] = a1;
+        for (int u = 0; u < U; ++u) x = fmaf(p[u], v[u][i / VW].get(i % VW), x);
+        acc[h][i] = x;
       }
       m[h] = mt;
     }
@@ -172,7 +194,7 @@ __device__ __forceinline__ void scan_range(const ActT *__restrict__ query, std::
   // Combine the four row-groups of the wave (lanes r, r^16, r^32, r^48 own
   // the same dims).
 #pragma unroll
-  for (int h = 0; h < NH; ++h) {
+  for (int h = 0; h < kGroup; ++h) {
     float mm = fmaxf(m[h], xor16(m[h]));
     mm = fmaxf(mm, xor32(mm));
     const float w = m[h] == -INFINITY ? 0.f : exp2f(m[h] - mm);
@@ -180,11 +202,11 @@ __device__ __forceinline__ void scan_range(const ActT *__restrict__ query, std::
     lw += xor16(lw);
     lw += xor32(lw);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      float a = acc[h][i] * w;
-      a += xor16(a);
-      a += xor32(a);
-      acc[h][i] = a;
+    for (int i = 0; i < kPerLane; ++i) {
+      float x = acc[h][i] * w;
+      x += xor16(x);
+      x += xor32(x);
+      acc[h][i] = x;
     }
     if (lane == 0) {
       sh.m[wave][h] = mm;
@@ -192,18 +214,15 @@ __device__ __forceinline__ void scan_range(const ActT *__restrict__ query, std::
     }
     if (lane < 16) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        sh.acc[wave][h][8 * r + i] = acc[h][i];
-        sh.acc[wave][h][128 + 8 * r + i] = acc[h][8 + i];
-      }
+      for (int i = 0; i < kPerLane; ++i) sh.acc[wave][h][16 * VW * (i / VW) + VW * r + i % VW] = acc[h][i];
     }
   }
 }
 
-// Merges the per-wave states of `sh` for output element (h, d): returns the
-// exp2-domain max, the sum and the unnormalised accumulator.
-template <int NH, int WAVES>
-__device__ __forceinline__ void combine_waves(const ScanShared<NH, WAVES> &sh, int h, int d,
+// Merges the per-wave states of `sh` for output element (h, d of the slice):
+// returns the exp2-domain max, the sum and the unnormalised accumulator.
+template <int DS, int WAVES>
+__device__ __forceinline__ void combine_waves(const ScanShared<DS, WAVES> &sh, int h, int d,
                                               float &m_out, float &l_out, float &a_out) {
   float mm = -INFINITY;
 #pragma unroll
@@ -219,6 +238,17 @@ __device__ __forceinline__ void combine_waves(const ScanShared<NH, WAVES> &sh, i
   m_out = mm;
   l_out = l;
   a_out = a;
+}
+
+// Stores the new token's K and V rows of kv_head at `pos`, cast to the cache
+// dtype (round to nearest even).
+template <typename ActT, typename CacheT>
+__device__ __forceinline__ void append_rows(const ScanArgs<ActT, CacheT> &a, std::size_t kv_head, std::size_t pos) {
+  if (threadIdx.x >= kHeadDim) return;
+  const std::size_t row = cache_row(a.head_major, pos, kv_head, a.max_ctx) + threadIdx.x;
+  const std::size_t src = kv_head * kHeadDim + threadIdx.x;
+  Elem<CacheT>::store(a.cache, row, Elem<ActT>::load(a.key_new, src));
+  Elem<CacheT>::store(a.cache, a.max_ctx * kKvHeads * kHeadDim + row, Elem<ActT>::load(a.value_new, src));
 }
 
 // sigmoid(x) = 1 / (1 + 2^(-x log2 e)) with the hardware exp2 and reciprocal

@@ -885,6 +885,36 @@ constexpr int kLdC = kChunk + 4;   // LDS row stride for 64-wide rows
 // Batched staging of a 64 x 128 block of rows (rows >= L repeat row L-1): thread owns
 // rows (tid + 256 r) / 16, dims 8 * ((tid + 256 r) % 16), r = 0..3, so every
 // global load of the block is issued before any of them is consumed.
+template <typename T> struct Chunk8;
+template <> struct Chunk8<bf16_bits> {
+  u32x4 w;
+  __device__ __forceinline__ void load(const bf16_bits *p) {
+    w = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+  }
+  __device__ __forceinline__ void zero() { w = u32x4{0u, 0u, 0u, 0u}; }
+  __device__ __forceinline__ float get(int i) const {
+    const std::uint32_t x = w[i >> 1];
+    return (i & 1) ? bf16_hi(x) : bf16_lo(x);
+  }
+};
+template <> struct Chunk8<float> {
+  float4 a, b;
+  __device__ __forceinline__ void load(const float *p) {
+    a = reinterpret_cast<const float4 *>(p)[0];
+    b = reinterpret_cast<const float4 *>(p)[1];
+  }
+  __device__ __forceinline__ void zero() {
+    a = make_float4(0.f, 0.f, 0.f, 0.f);
+    b = a;
+  }
+  __device__ __forceinline__ float get(int i) const {
+    switch (i) {
+    case 0: return a.x; case 1: return a.y; case 2: return a.z; case 3: return a.w;
+    case 4: return b.x; case 5: return b.y; case 6: return b.z; default: return b.w;
+    }
+  }
+};
+
 template <typename T> struct RowBlock {
   Chunk8<T> c[4];
   template <typename Addr>

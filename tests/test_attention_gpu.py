@@ -545,3 +545,20 @@ def test_batched_ragged_decode_cfg4_full_size(gpu):
         keys, vals = c[0].transpose(1, 0, 2), c[1].transpose(1, 0, 2)
         expect = orc.attention_core(from_dev(q[b])[None], keys, vals, from_dev(g[b])[None], L - 1)[0]
         assert_bf16_close(got[b], expect, what=f"cfg4 seq {b} len {L} vs oracle")
+
+
+@pytest.mark.parametrize("act,cdt", [(1, 0), (1, 1), (3, 0)])
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("ctx,max_ctx,mode", [(1, 300, 2), (15, 300, 2), (255, 300, 2), (256, 300, 2), (257, 300, 2),
+                                              (1000, 4096, 0), (3000, 4096, 0), (6200, 8192, 2), (12345, 16384, 2),
+                                              (700, 1024, 3), (700, 1024, 1)])
+def test_scan_decode_slices(gpu, act, cdt, layout, ctx, max_ctx, mode):
+    # The f32-activation / f32-cache kernels: single-block and partition work in one launch, one to four dims slices
+    # per partition (plans of up to 24, 48 and more partitions), the new row in a partition's first, last and only
+    # place, host and device positions.
+    for device_position in (False, True):
+        out, expect, cache, keys, vals, _, _ = run_decode(act, cdt, layout, ctx, max_ctx, mode=mode,
+                                                          device_position=device_position, seed=ctx + layout)
+        assert close_enough(out, expect), (device_position,)
+        ck, cv = read_cache(cache, layout, ctx, max_ctx)
+        assert np.array_equal(ck, keys) and np.array_equal(cv, vals)
