@@ -621,8 +621,9 @@ __global__ __launch_bounds__(WAVES * 64) void decode_dynamic_mfma_kernel(
 // of 3000 tokens had 48 workgroups, and a step was four launches (append, early
 // exit of the single-block kernel, partitions, merge): 26.5 us on an f32
 // token-major cache, 15 of them the partitions.  Sliced, with the append and the
-// choice of path inside, it is two launches and 15.8 us (partitions 11.4: 320 KiB of
-// plain loads per CU at about 33 B/clk, then their FMAs).
+// choice of path inside, it is two launches and 16.0 us, 11.4 to 12.5 of them the
+// partitions: with four slices they read 61 MB (K four times, V once; 25 MB are
+// the cache's own) and repeat the scores four times on the vector units.
 constexpr int kScanWaves = 8;
 constexpr int scan_unroll(int ds) { return ds == 1 ? 2 : 4; } // tokens per row-group and step (registers)
 
