@@ -1583,21 +1583,30 @@ __global__ __launch_bounds__(256) void chunk_scan_kernel(ChunkScratch scratch,
 // T = (I + A)^-1, and the record (Tb split, M split, G).
 // kSplit: q and k arrive as (hi, lo) bf16 planes (fp32 values split), and
 // each product is formed as hi*hi + hi*lo + lo*hi.
+//
+// A workgroup is a chain of latencies (rows in, products, three dependent steps
+// of the inverse, records out), so what bounds the kernel is how many of them a
+// CU holds.  Q is read by the wave that multiplies it, M leaves from registers,
+// and A, T and Y take K's place once every wave has read it: 39 KiB, where
+// all of them side by side were 127 KiB and one workgroup per CU.
+// At 4001 tokens (2016 workgroups) 72 -> 42 us.  Three per CU in the split
+// form by its 143 registers: a fourth would spill.
 template <bool kSplit> struct TbShared {
-  bf16_bits k[kSplit ? 2 : 1][kChunk][kChunkDim + 8];
-  bf16_bits q[kSplit ? 2 : 1][kChunk][kChunkDim + 8];
-  float a[kChunk][kLdC];
-  float tm[kChunk][kLdC];
-  float mm[kChunk][kLdC];
-  float y[32][36];
+  union {
+    bf16_bits k[kSplit ? 2 : 1][kChunk][kChunkDim + 8];
+    struct {
+      float a[kChunk][kLdC];
+      float tm[kChunk][kLdC];
+      float y[32][36];
+    };
+  };
   float g[kChunk];
   float beta[kChunk];
 };
 
-// Writes a [64][64] fp32 LDS tile (times the per-column factor col[j] when
-// kCol) to a record as split bf16 [2][64][64]: thread -> row tid / 4,
-// columns 16 (tid % 4) .. +15.  All LDS reads go out before the first use.
-template <bool kCol>
+// Writes a [64][64] fp32 LDS tile times the per-column factor col[j] to a
+// record as split bf16 [2][64][64]: thread -> row tid / 4, columns
+// 16 (tid % 4) .. +15.  All LDS reads go out before the first use.
 __device__ __forceinline__ void write_split_64(const float (*src)[kLdC], const float *col, bf16_bits *dst) {
   const int i = threadIdx.x >> 2, j0 = 16 * (threadIdx.x & 3);
   float v[16];
@@ -1609,15 +1618,13 @@ __device__ __forceinline__ void write_split_64(const float (*src)[kLdC], const f
     v[4 * e + 2] = x.z;
     v[4 * e + 3] = x.w;
   }
-  if constexpr (kCol) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float4 c = *reinterpret_cast<const float4 *>(&col[j0 + 4 * e]);
-      v[4 * e] *= c.x;
-      v[4 * e + 1] *= c.y;
-      v[4 * e + 2] *= c.z;
-      v[4 * e + 3] *= c.w;
-    }
+  for (int e = 0; e < 4; ++e) {
+    const float4 c = *reinterpret_cast<const float4 *>(&col[j0 + 4 * e]);
+    v[4 * e] *= c.x;
+    v[4 * e + 1] *= c.y;
+    v[4 * e + 2] *= c.z;
+    v[4 * e + 3] *= c.w;
   }
   u32x4 hi[2], lo[2];
 #pragma unroll
@@ -1635,14 +1642,15 @@ __device__ __forceinline__ void write_split_64(const float (*src)[kLdC], const f
 }
 
 template <bool kSplit>
-__global__ __launch_bounds__(256) void chunk_tb_kernel(Src<bf16_bits> qs, Src<bf16_bits> ks, std::size_t lo_plane,
+__global__ __launch_bounds__(256, 3) void chunk_tb_kernel(Src<bf16_bits> qs, Src<bf16_bits> ks, std::size_t lo_plane,
                                                        const float *__restrict__ beta,
                                                        const float *__restrict__ gdecay,
                                                        ChunkScratch scratch, std::size_t tokens,
                                                        std::size_t hk, std::size_t hv) {
   constexpr int kHalves = kSplit ? 2 : 1;
   __shared__ TbShared<kSplit> sh;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lk = lane >> 4;
   const std::size_t h = blockIdx.x;
   const std::size_t kh = h % hk;
@@ -1650,18 +1658,26 @@ __global__ __launch_bounds__(256) void chunk_tb_kernel(Src<bf16_bits> qs, Src<bf
   const int L = static_cast<int>(tokens - t0 < kChunk ? tokens - t0 : kChunk);
   unsigned char *record = scratch.at(h, blockIdx.y);
 
-  // K and Q rows (each plane): item tid + 256 r -> row item / 16, dims
-  // 8 (item % 16) .. +7; rows past L repeat row L-1.
-  u32x4 kv[kHalves][4], qv[kHalves][4];
+  // K rows (each plane): item tid + 256 r -> row item / 16, dims
+  // 8 (item % 16) .. +7; Q row 16 w + lr of wave w as its product reads it.
+  // Rows past L repeat row L-1.
+  u32x4 kv[kHalves][4];
+  bf16x8 qrow[kHalves][4];
 #pragma unroll
   for (int hl = 0; hl < kHalves; ++hl)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int p = tid + 256 * r, i = p >> 4, d = 8 * (p & 15);
-      const std::size_t t = t0 + (i < L ? i : L - 1);
-      kv[hl][r] = *reinterpret_cast<const u32x4 *>(src_row(ks, t, kh, d) + hl * lo_plane);
-      qv[hl][r] = *reinterpret_cast<const u32x4 *>(src_row(qs, t, kh, d) + hl * lo_plane);
+      kv[hl][r] = *reinterpret_cast<const u32x4 *>(src_row(ks, t0 + (i < L ? i : L - 1), kh, d) + hl * lo_plane);
     }
+  {
+    const int i = 16 * wave + lr;
+    const bf16_bits *qr = src_row(qs, t0 + (i < L ? i : L - 1), kh, 8 * lk);
+#pragma unroll
+    for (int hl = 0; hl < kHalves; ++hl)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) qrow[hl][n] = *reinterpret_cast<const bf16x8 *>(qr + hl * lo_plane + 32 * n);
+  }
   float bt = 0.f, gt = 0.f;
   if (tid < L) {
     bt = beta[(t0 + tid) * hv + h];
@@ -1673,88 +1689,96 @@ __global__ __launch_bounds__(256) void chunk_tb_kernel(Src<bf16_bits> qs, Src<bf
     for (int r = 0; r < 4; ++r) {
       const int p = tid + 256 * r, i = p >> 4, d = 8 * (p & 15);
       *reinterpret_cast<u32x4 *>(&sh.k[hl][i][d]) = kv[hl][r];
-      *reinterpret_cast<u32x4 *>(&sh.q[hl][i][d]) = qv[hl][r];
     }
-  if (tid < kChunk) {
-    sh.beta[tid] = bt;
-    sh.g[tid] = gt;
+  // G: wave 0 holds g of every row (rows past L repeat G[L-1]: their g is 0)
+  if (wave == 0) {
+    sh.beta[lane] = bt;
+    sh.g[lane] = wave_prefix_sum(gt);
   }
   __syncthreads();
-  if (wave == 0) sh.g[lane] = wave_prefix_sum(sh.g[lane]); // rows past L repeat G[L-1] (g = 0)
-  __syncthreads();
   // A and M: wave w takes row tile w and column tiles 0 .. w (tiles right of
-  // the diagonal are 0).
+  // the diagonal are 0).  A is formed as rows x columns, M transposed, so that a
+  // lane has four consecutive columns of a row of M to store: row 16 w + lr,
+  // columns 16 tj + 4 lk .. +3.
+  floatx4 at[4];
   {
     const float kk_scale = ks.scale * ks.scale, qk_scale = qs.scale * ks.scale;
+    const int mi = 16 * wave + lr;
+    const float gm = sh.g[mi];
     float gi[4], bi[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       gi[r] = sh.g[16 * wave + 4 * lk + r];
       bi[r] = sh.beta[16 * wave + 4 * lk + r] * kk_scale;
     }
-    bf16x8 krow[kHalves][4], qrow[kHalves][4];
+    bf16x8 krow[kHalves][4];
 #pragma unroll
     for (int hl = 0; hl < kHalves; ++hl)
 #pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        krow[hl][n] = lds8(&sh.k[hl][16 * wave + lr][32 * n + 8 * lk]);
-        qrow[hl][n] = lds8(&sh.q[hl][16 * wave + lr][32 * n + 8 * lk]);
-      }
-    floatx4 diag = floatx4{}; // this lane's part of A's diagonal tile (w, w)
+      for (int n = 0; n < 4; ++n) krow[hl][n] = lds8(&sh.k[hl][16 * wave + lr][32 * n + 8 * lk]);
+    bf16_bits *m_row = reinterpret_cast<bf16_bits *>(record + rec2::kM) + mi * kChunk + 4 * lk;
+#pragma unroll
     for (int tj = 0; tj < 4; ++tj) {
-      const int j = 16 * tj + lr;
-      if (tj > wave) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sh.mm[16 * wave + 4 * lk + r][j] = 0.f;
-        continue;
-      }
-      bf16x8 kcol[kHalves][4];
-#pragma unroll
-      for (int hl = 0; hl < kHalves; ++hl)
-#pragma unroll
-        for (int n = 0; n < 4; ++n) kcol[hl][n] = lds8(&sh.k[hl][16 * tj + lr][32 * n + 8 * lk]);
-      floatx4 aa = floatx4{}, am = floatx4{};
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        aa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(krow[0][n], kcol[0][n], aa, 0, 0, 0);
-        am = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qrow[0][n], kcol[0][n], am, 0, 0, 0);
-      }
-      if constexpr (kSplit) {
-        // hi*lo and lo*hi terms (lo*lo is below 2^-16 of the product).
-        floatx4 aa2 = floatx4{}, am2 = floatx4{};
+      at[tj] = floatx4{};
+      u32x2 mh = {}, ml = {};
+      if (tj <= wave) { // (uniform)
+        floatx4 aa = floatx4{}, am = floatx4{}, aa2 = floatx4{}, am2 = floatx4{};
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
-          aa2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(krow[0][n], kcol[kHalves - 1][n], aa2, 0, 0, 0);
-          am2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qrow[0][n], kcol[kHalves - 1][n], am2, 0, 0, 0);
-          aa2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(krow[kHalves - 1][n], kcol[0][n], aa2, 0, 0, 0);
-          am2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qrow[kHalves - 1][n], kcol[0][n], am2, 0, 0, 0);
+          const bf16x8 kc = lds8(&sh.k[0][16 * tj + lr][32 * n + 8 * lk]);
+          aa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(krow[0][n], kc, aa, 0, 0, 0);
+          am = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc, qrow[0][n], am, 0, 0, 0);
+          if constexpr (kSplit) {
+            // hi*lo and lo*hi terms (lo*lo is below 2^-16 of the product).
+            const bf16x8 kl = lds8(&sh.k[kHalves - 1][16 * tj + lr][32 * n + 8 * lk]);
+            aa2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(krow[0][n], kl, aa2, 0, 0, 0);
+            am2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qrow[0][n], am2, 0, 0, 0);
+            aa2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(krow[kHalves - 1][n], kc, aa2, 0, 0, 0);
+            am2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kc, qrow[kHalves - 1][n], am2, 0, 0, 0);
+          }
         }
-        aa += aa2;
-        am += am2;
-      }
-      const float gj = sh.g[j];
+        if constexpr (kSplit) {
+          aa += aa2;
+          am += am2;
+        }
+        const int j = 16 * tj + lr;
+        const float gj = sh.g[j];
+        const floatx4 gc = *reinterpret_cast<const floatx4 *>(&sh.g[16 * tj + 4 * lk]);
+        float mv[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = 16 * wave + 4 * lk + r;
-        const float e = __expf(gi[r] - gj);
-        const float av = (j < i && i < L) ? bi[r] * e * aa[r] : 0.f;
-        sh.a[i][j] = av;
-        if (tj == wave) diag[r] = av;
-        sh.mm[i][j] = (j <= i && i < L) ? qk_scale * e * am[r] : 0.f;
+        for (int r = 0; r < 4; ++r) {
+          const int i = 16 * wave + 4 * lk + r;
+          at[tj][r] = (j < i && i < L) ? bi[r] * __expf(gi[r] - gj) * aa[r] : 0.f;
+          mv[r] = (16 * tj + 4 * lk + r <= mi && mi < L) ? qk_scale * __expf(gm - gc[r]) * am[r] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          std::uint32_t hw, lw;
+          split2(mv[2 * e], mv[2 * e + 1], hw, lw);
+          mh[e] = hw;
+          ml[e] = lw;
+        }
       }
+      *reinterpret_cast<u32x2 *>(m_row + 16 * tj) = mh;
+      *reinterpret_cast<u32x2 *>(m_row + kChunk * kChunk + 16 * tj) = ml;
     }
-    // Step 1 of the inverse straight from the registers: A[16w + r][16w + j]
-    // is element r % 4 of lane 16 (r / 4) + j.
-    invert_step1(sh.tm, wave, [&](int r, int j) {
-      return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(diag[r & 3]), 16 * (r >> 2) + j));
-    });
   }
-  __syncthreads();
-  // M and G are final here: their record stores drain during the inverse.
-  write_split_64<false>(sh.mm, nullptr, reinterpret_cast<bf16_bits *>(record + rec2::kM));
   if (tid < kChunk) reinterpret_cast<float *>(record + rec2::kG)[tid] = sh.g[tid];
+  __syncthreads(); // K has been read: A, T and Y take its place
+#pragma unroll
+  for (int tj = 0; tj < 4; ++tj)
+    if (tj <= wave)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sh.a[16 * wave + 4 * lk + r][16 * tj + lr] = at[tj][r];
+  const floatx4 diag = wave == 0 ? at[0] : wave == 1 ? at[1] : wave == 2 ? at[2] : at[3]; // tile (w, w) of A
+  // Step 1 of the inverse straight from the registers: A[16w + r][16w + j]
+  // is element r % 4 of lane 16 (r / 4) + j.
+  invert_step1(sh.tm, wave, [&](int r, int j) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(diag[r & 3]), 16 * (r >> 2) + j));
+  });
+  __syncthreads();
   invert_steps23(sh.a, sh.tm, sh.y);
-  write_split_64<true>(sh.tm, sh.beta, reinterpret_cast<bf16_bits *>(record + rec2::kTb));
+  write_split_64(sh.tm, sh.beta, reinterpret_cast<bf16_bits *>(record + rec2::kTb));
 }
 
 // Operands of one chunk, staged in LDS by LDS-direct loads.  Q and K rows use
