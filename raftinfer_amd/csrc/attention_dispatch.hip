@@ -3,9 +3,10 @@
 //
 // Host semantics follow cpp/kernels/qwen35_attention.cu:103-613 and
 // cpp/kernels/qwen35_online_attention.cu:27-94, :1145-1218.  The online
-// prefill runs the bf16 MFMA kernel (attention_prefill_mfma.hip) for the
-// Qwen3.5 signature with bf16 activations and cache, and a generic fp32
-// wave-per-row kernel for every other supported shape / dtype / layout.
+// prefill runs on bf16 MFMA for the Qwen3.5 signature with bf16 activations
+// (attention_prefill_mfma.hip, attention_prefill_wide.hip; f32 caches by
+// three-way split values), and a generic fp32 wave-per-row kernel for every
+// other supported shape / dtype / layout.
 #include <cmath>
 #include "decode_scan.hpp"
 #include "prefill_mfma.hpp"
