@@ -24,6 +24,12 @@
 //     Barriers and loads bound NB = 1 (128 KiB per round of 4 tiles: 1.4 us),
 //     the card's power NB = 2 (2048 tokens behind 30000: 1.2 PFLOP/s, the rate
 //     that a bf16 matrix product of 8192^3 reaches here).
+//   - a masked key has probability 0, and 0 times an infinite or NaN value is not 0:
+//     with NB = 2, a workgroup whose own tokens have such values throws its sums away
+//     and forms them again, the tiles that mask key by key (careful_tile).  With 8
+//     tokens per workgroup (here and in prefill_mfma_kernel) such a value reaches the
+//     up to seven tokens before it in its workgroup; the look for them would take
+//     0.8 of 54 us there (512 tokens behind 3584).
 // prefill_plan (attention_prefill_mfma.hip) says which form takes a call.
 #include "prefill_mfma.hpp"
 #include "prefill_tile.hpp"
@@ -167,6 +173,178 @@ __device__ __forceinline__ float lds_read_f1(unsigned addr) {
   return *(const __attribute__((address_space(3))) float *)(std::uintptr_t)(addr);
 }
 template <bool F32> using CacheElem = std::conditional_t<F32, float, bf16_bits>;
+
+// The output of a workgroup's tile (kTok query tokens of one KV head, as
+// prefill_wide_kernel deals them) where its own tokens have infinite or NaN values:
+// one column block (4 heads x 8 tokens) per wave over all keys, a 32-key tile at a
+// time in the wave's own part of LDS (K and V rows of 512 bytes, 16-byte chunk c of
+// row r at c ^ swz(r)), the tiles that mask key by key.  A chain of latencies, about
+// 3.4 us a tile (6001 tokens, every value NaN: 1.27 ms in place of 0.34).  It derives
+// everything anew and is not the streaming loop run again: values kept for either
+// took registers in the streaming loop and its ends (6001 tokens of finite values:
+// 308 us, 313 to 318 with a second run of the loop, 449 with the Q operands kept).
+template <int kTok, bool HeadMajor, bool FromInput, bool NormQ>
+__device__ __forceinline__ void careful_tile(const bf16_bits *query, const bf16_bits *key_in, const bf16_bits *value_in,
+                                             const bf16_bits *gate, bf16_bits *output, const bf16_bits *cache,
+                                             std::size_t tokens, std::size_t max_ctx, std::size_t past,
+                                             const PrefillNormRope &nq, unsigned lds0) {
+  int tid = threadIdx.x;
+  unsigned block = blockIdx.x;
+  asm volatile("" : "+v"(tid), "+s"(block)); // (nothing of this is formed before the streaming loop)
+  const int lane = tid & 63, col = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (wave >= kTok / 8) return;
+  const std::size_t qtile = ceil_div_u(tokens, kTok) - 1 - (2 * (block >> 3) + (block & 1u));
+  const std::size_t kv_head = (block & 7u) >> 1, t0 = qtile * kTok;
+  const std::size_t q_rows = tokens - t0 < kTok ? tokens - t0 : kTok, key_end = past + t0 + q_rows;
+  // Token slot and head of row r (0..31) of the wave's block.
+  auto slot = [&](int r) __attribute__((always_inline)) {
+    const std::size_t tt = 8 * wave + (r & 7);
+    return tt < q_rows ? tt : q_rows - 1;
+  };
+  auto io_row = [&](int r) __attribute__((always_inline)) {
+    return ((t0 + slot(r)) * kQueryHeads + kv_head * kGroup + (r >> 3)) * kHeadDim;
+  };
+  const unsigned k_at = lds0 + 40960u * wave, v_at = k_at + 16384u;
+  constexpr std::size_t q_row_elems = NormQ ? 2 * kHeadDim : kHeadDim;
+  // ---- Q rows in the place of K, normalised there, then in registers
+#pragma unroll 1
+  for (int i = 0; i < 16; ++i) {
+    const int r = 2 * i + half;
+    load_lds_b128(query + (t0 * kQueryHeads + kv_head * kGroup) * q_row_elems,
+                  static_cast<std::uint32_t>(slot(r) * kQueryHeads + (r >> 3)) * (q_row_elems * 2) + 16u * (col ^ swz(r)),
+                  k_at + 1024u * i);
+  }
+  if constexpr (NormQ) { // weight and rotation tables in the place of V
+    const std::uint32_t bytes = nq.weight_f32 ? 1024u : 512u;
+    load_lds_b128(nq.weight, 16u * lane < bytes ? 16u * lane : bytes - 16u, v_at);
+    auto rot = reinterpret_cast<float(*)[kHeadDim]>(lds_ptr<float>(v_at + 1024u));
+    for (int i = lane; i < 8 * nq.pairs; i += kWave) {
+      const int s = i / nq.pairs, pp = i - s * nq.pairs;
+      float cs, sn;
+      rope_cos_sin(pp, past + t0 + slot(s), nq.ratio, cs, sn);
+      rot[s][pp] = cs;
+      rot[s][nq.pairs + pp] = sn;
+    }
+    wait_vm<0>();
+    wave_lds_order();
+    const float *weight = lds_ptr<float>(v_at);
+#pragma unroll 1
+    for (int h = 0; h < 4; ++h) { // the 8 token slots of a head
+      bf16_bits *staged = lds_ptr<bf16_bits>(k_at + 4096u * h);
+      if (nq.pairs % 32 == 0)
+        norm_rope_rows_sliced(staged, lane >> 3, lane & 7, weight, nq.weight_f32, nq.pairs, rot[lane >> 3], nq.epsilon);
+      else
+        norm_rope_rows_lanewise(staged, 0, lane, weight, nq.weight_f32, nq.pairs, rot, nq.epsilon);
+    }
+    wave_lds_order();
+  }
+  wait_vm<0>();
+  const unsigned k_lane = k_at + col * 512u + 16u * (half ^ swz(col)); // chunk 2 kk + half: exclusive-or 32 kk
+  bf16x8 q[16];
+#pragma unroll
+  for (int kk = 0; kk < 16; ++kk) q[kk] = lds_read_b128(k_lane ^ (32u * kk));
+  // V^T operand of dims block nb, key step kb: as in prefill_wide_kernel
+  const int vg = (lane >> 4) & 1, vr = lane & 15, vrow = 4 * half + (vr >> 2);
+  const unsigned v_lane = v_at + vrow * 512u + 16u * ((2 * vg + ((vr & 3) >> 1)) ^ swz(vrow)) + 8u * (vr & 1);
+  constexpr std::uint32_t row_bytes = (HeadMajor && !FromInput ? kHeadDim : kKvHeads * kHeadDim) * 2;
+  const bf16_bits *k_src = FromInput ? key_in + kv_head * kHeadDim : cache + cache_row(HeadMajor, 0, kv_head, max_ctx);
+  const bf16_bits *v_src = FromInput ? value_in + kv_head * kHeadDim : k_src + max_ctx * kKvHeads * kHeadDim;
+  const float scale = kLog2e / 16.0f;
+  const std::ptrdiff_t pos = static_cast<std::ptrdiff_t>(past + t0 + slot(col));
+  acc_fence();
+  static_for<128>([&](auto i) __attribute__((always_inline)) { acc_set<i>(0.f); });
+  float m_run = -INFINITY, l_run = 0.f;
+#pragma unroll 1
+  for (std::size_t k0 = 0; k0 < key_end; k0 += kKTile) {
+    const std::uint32_t last = static_cast<std::uint32_t>(key_end - 1 - k0 < 31 ? key_end - 1 - k0 : 31);
+    wait_lgkm0(); // the last tile has been read
+#pragma unroll 1
+    for (int i = 0; i < 16; ++i) {
+      const std::uint32_t r = 2 * i + half, voff = (r < last ? r : last) * row_bytes + 16u * (col ^ swz(r));
+      load_lds_b128(k_src + k0 * (row_bytes / 2), voff, k_at + 1024u * i);
+      load_lds_b128(v_src + k0 * (row_bytes / 2), voff, v_at + 1024u * i);
+    }
+    wait_vm<0>();
+    floatx16 s;
+    static_for<16>([&](auto kk) __attribute__((always_inline)) {
+      bf16x8 a = lds_read_b128(k_lane ^ (32u * kk));
+      asm volatile("s_nop 1" : "+v"(a)); // (wait states before the MFMA)
+      if constexpr (kk == 0) s_mfma_zero(s, a, q[kk]); else s_mfma(s, a, q[kk]);
+    });
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(s));
+    const std::ptrdiff_t lim = pos - static_cast<std::ptrdiff_t>(k0); // last visible key
+    float x[16], top = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      x[i] = (i >> 2) * 8 + 4 * half + (i & 3) > lim ? -INFINITY : s[i] * scale;
+      top = fmaxf(top, x[i]);
+    }
+    top = max_xor32(top);
+    const bool grow = top > m_run + kLazyRescale;
+    if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+      const float sc = grow ? fexp2(m_run - top) : 1.0f;
+      l_run *= sc;
+      m_run = grow ? top : m_run;
+      static_for<128>([&](auto i) __attribute__((always_inline)) { acc_set<i>(acc_get<i>() * sc); });
+    }
+    const float m_ref = m_run == -INFINITY ? 0.f : m_run;
+    std::uint32_t p[8]; // P^T, bf16 pairs in accumulator order
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      p[i] = pack_bf16x2(fexp2(x[2 * i] - m_ref), fexp2(x[2 * i + 1] - m_ref));
+      l_run = dot2_bf16(p[i], 0x3F803F80u, l_run);
+    }
+    acc_fence();
+    if (k0 + kKTile - 1 <= past + t0) {
+      static_for<16>([&](auto st) __attribute__((always_inline)) {
+        constexpr int kb = st & 1, nb = st >> 1;
+        const unsigned a = (v_lane ^ (64u * nb)) + 8192u * kb;
+        const u32x2 lo = lds_read_tr16(a), hi = lds_read_tr16(a + 4096u);
+        bf16x8 v = __builtin_bit_cast(bf16x8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+        bf16x8 w = __builtin_bit_cast(bf16x8, u32x4{p[4 * kb], p[4 * kb + 1], p[4 * kb + 2], p[4 * kb + 3]});
+        asm volatile("s_nop 1" : "+v"(v), "+v"(w));
+        acc_mfma<nb>(v, w);
+      });
+    } else {
+#pragma unroll 1
+      for (int key = 0; key < kKTile; ++key) {
+        std::uint32_t pair = p[0]; // the key's probability, in the lanes of its half, then in the whole column
+#pragma unroll
+        for (int i = 1; i < 8; ++i) {
+          pair = i == 2 * (key >> 3) + ((key & 3) >> 1) ? p[i] : pair;
+          asm volatile("" : "+v"(pair)); // a chain of selects, not an array in scratch
+        }
+        float w = (key & 1) != 0 ? bf16_hi(pair) : bf16_lo(pair);
+        const float other = xor32(w);
+        w = ((key >> 2) & 1) != half ? other : w;
+        const unsigned row = v_at + key * 512u;
+        static_for<32>([&](auto quad) __attribute__((always_inline)) { // dims 8 quad + 4 half .. +3
+          const u32x2 y = *lds_ptr<u32x2>(row + 16u * (quad ^ swz(key)) + 8u * half);
+          static_for<4>([&](auto e) __attribute__((always_inline)) {
+            const float v = (e & 1) != 0 ? bf16_hi(y[e >> 1]) : bf16_lo(y[e >> 1]);
+            const float was = acc_get<4 * quad + e>();
+            acc_set<4 * quad + e>(key <= lim ? fmaf(w, v, was) : was);
+          });
+        });
+        acc_fence();
+      }
+    }
+    mfma_drain();
+  }
+  const float inv = 1.0f / (l_run + xor32(l_run));
+  const bf16_bits *gate_row = NormQ ? query + 2 * io_row(col) + kHeadDim : gate + io_row(col);
+  if (static_cast<std::size_t>(8 * wave + (col & 7)) >= q_rows) return;
+  static_for<32>([&](auto quad) __attribute__((always_inline)) {
+    constexpr int d = 8 * quad;
+    const u32x2 g = *reinterpret_cast<const u32x2 *>(gate_row + d + 4 * half);
+    *reinterpret_cast<u32x2 *>(output + io_row(col) + d + 4 * half) =
+        u32x2{pack_bf16x2(acc_get<4 * quad>() * inv * sigmoid_gate(bf16_lo(g[0])),
+                          acc_get<4 * quad + 1>() * inv * sigmoid_gate(bf16_hi(g[0]))),
+              pack_bf16x2(acc_get<4 * quad + 2>() * inv * sigmoid_gate(bf16_lo(g[1])),
+                          acc_get<4 * quad + 3>() * inv * sigmoid_gate(bf16_hi(g[1])))};
+  });
+}
 
 template <int NB, int KS, bool HeadMajor, bool FromInput, bool NormQ, bool F32 = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_wide_kernel(
@@ -929,6 +1107,30 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
                                                 ((t0 + tt) * kKvHeads + kv_head) * kHeadDim + 8 * piece);
     }
   }
+  auto store_app = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < kApp; ++j) {
+      int pl, tok, piece;
+      app_at(j, pl, tok, piece);
+      if (static_cast<std::size_t>(tok) < q_rows)
+        *reinterpret_cast<u32x4 *>(cache + pl * plane + cache_row(HeadMajor, t0 + tok, kv_head, max_ctx) + 8 * piece) =
+            app[j];
+    }
+  };
+  // Pieces of the V rows that some of the tile's columns must not see, or that are
+  // read again in the place of rows past the last (with FromInput the V half of app).
+  constexpr bool kWatch = NB == 2;
+  constexpr int kOwn = kWatch && !FromInput ? kTok / 8 : 1;
+  [[maybe_unused]] u32x4 own[kOwn];
+  if constexpr (kWatch && !FromInput) {
+#pragma unroll
+    for (int j = 0; j < kOwn; ++j) {
+      const std::size_t idx = kWave * wave + lane_e + kThreads * j, tt = idx >> 5 == 0 ? 1 : idx >> 5;
+      own[j] = *reinterpret_cast<const u32x4 *>(base_of(v_src, past + t0 + (tt < q_rows ? tt : q_rows - 1)) +
+                                                16 * (idx & 31));
+    }
+  }
+  bool again = false; // one of them is an infinity or a NaN
   // Partials of wave (g, cg) for the finisher of part q (q != g): [dims block of
   // the part][register quad][lane] float4; its (max, sum) of each block, [2 NB][lane].
   constexpr unsigned kPartBytes = P::kParts * 4 * kWave * sizeof(float4);
@@ -937,6 +1139,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   };
   auto ml_at = [&](int g) __attribute__((always_inline)) {
     return lds_ptr<float>(lds0 + g * P::kArea + (kShare == 1 ? g * kPartBytes : 2 * kPartBytes + cg * 1024u));
+  };
+  auto flag_at = [&](int w) __attribute__((always_inline)) { // what wave w found in its pieces
+    return lds_ptr<unsigned>(lds0 + (w % KS) * P::kArea + (kShare == 1 ? w % KS : 2) * kPartBytes + 4096u + 4u * (w / KS));
   };
   static_for<NB>([&](auto bc) __attribute__((always_inline)) {
     constexpr int b = bc;
@@ -964,6 +1169,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         ml_at(kg)[(2 * bb) * kWave + lane_e] = m_run[bb];
         ml_at(kg)[(2 * bb + 1) * kWave + lane_e] = l_run[bb];
       }
+      if constexpr (kWatch) {
+        std::uint32_t bad = 0; // an exponent of all ones, plus one, carries into the sign's place
+        auto look = [&](const u32x4 &x) __attribute__((always_inline)) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bad |= ((x[e] & 0x7F807F80u) + 0x00800080u) & 0x80008000u;
+        };
+#pragma unroll
+        for (int j = 0; j < (FromInput ? kApp / 2 : kOwn); ++j)
+          if constexpr (FromInput) look(app[kApp / 2 + j]); else look(own[j]);
+        const unsigned any = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
+        if (lane_e == 0) *flag_at(wave) = any;
+      }
       wait_vm<0>(); // this wave's gate rows
     }
     __syncthreads();
@@ -983,6 +1200,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     for (int g = 0; g < KS; ++g) {
       mw[g] = ml_at(g)[(2 * b) * kWave + lane_e];
       lw[g] = ml_at(g)[(2 * b + 1) * kWave + lane_e];
+    }
+    if constexpr (b == 0 && kWatch) {
+      unsigned any = 0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) any |= *flag_at(w);
+      again = __builtin_amdgcn_readfirstlane(any) != 0;
     }
 #pragma unroll
     for (int g = 0; g < KS; ++g) mm = fmaxf(mm, mw[g]);
@@ -1031,19 +1254,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
 #pragma unroll
     for (int i = 0; i < 32 / kPerStore; ++i) {
       const int c = kPerStore * i + lane_e / kChunks, k = kChunks * kg + lane_e % kChunks, r = r0 + c;
-      if (static_cast<std::size_t>(8 * (r >> 5) + (r & 7)) < q_rows)
+      if (!again && static_cast<std::size_t>(8 * (r >> 5) + (r & 7)) < q_rows)
         *reinterpret_cast<u32x4 *>(output + io_row(r) + 8 * k) = *lds_ptr<u32x4>(row_at(r) + 16u * (k ^ swz(c)));
     }
   });
-  if constexpr (FromInput) {
-#pragma unroll
-    for (int j = 0; j < kApp; ++j) {
-      int pl, tok, piece;
-      app_at(j, pl, tok, piece);
-      if (static_cast<std::size_t>(tok) < q_rows)
-        *reinterpret_cast<u32x4 *>(cache + pl * plane + cache_row(HeadMajor, t0 + tok, kv_head, max_ctx) + 8 * piece) =
-            app[j];
-    }
+  if constexpr (FromInput) store_app();
+  if constexpr (kWatch) {
+    if (!again) return;
+    __syncthreads(); // the flags have been read
+    careful_tile<kTok, HeadMajor, FromInput, NormQ>(query, key_in, value_in, gate, output, cache, tokens, max_ctx, past, nq,
+                                                    lds0);
   }
 }
 

@@ -102,12 +102,14 @@ def test_fused_decode_against_oracle(gpu):
     assert_bf16_close(ck[ctx - 1], kb, what="appended k", both_bf16=True)
 
 
-def _prefill_case(T, past, rot, wdt, layout, seed):
+def _prefill_case(T, past, rot, wdt, layout, seed, edit_v=None):
     r = rng(seed)
     max_ctx = past + T
     pk, pv = bf16(normal(r, past, HKV, D)), bf16(normal(r, past, HKV, D))
     qg = bf16(normal(r, T, HQ, 2, D))
     kraw, v = bf16(normal(r, T, HKV, D)), bf16(normal(r, T, HKV, D))
+    if edit_v is not None:
+        edit_v(v)
     wq, wk = _norm_weights(r, wdt)
     base, eps = 1e7, 1e-6
     cache0 = to_dev(make_cache(pk, pv, layout, max_ctx), BF)

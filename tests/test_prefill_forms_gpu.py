@@ -13,12 +13,15 @@ from test_fused_gpu import _prefill_case
 pytestmark = pytest.mark.gpu
 
 
-def attend(T, past, layout, seed):
-    """Output, torch fp32 reference and cache (as written, [2][4][ctx][256]) of random inputs."""
+def attend(T, past, layout, seed, edit=None):
+    """Output, torch fp32 reference (non-finite values of V taken as 0) and whether the cache was written as expected,
+    for random inputs; edit(k, v) changes the rows [past + T][4][256] before the call."""
     g = torch.Generator(device="cuda").manual_seed(seed)
     rnd = lambda *shape: torch.randn(*shape, device="cuda", generator=g).to(torch.bfloat16)
     n = past + T
     q, gate, k, v = rnd(T, HQ, D), rnd(T, HQ, D), rnd(n, HKV, D), rnd(n, HKV, D)
+    if edit is not None:
+        edit(k, v)
     rows = torch.stack([k, v])  # token-major
     full = rows.clone()
     rows[:, past:] = 0
@@ -29,6 +32,7 @@ def attend(T, past, layout, seed):
     torch.cuda.synchronize()
     qf = q.float().permute(1, 0, 2)
     kf, vf = (x.float().repeat_interleave(HQ // HKV, dim=1).permute(1, 0, 2).contiguous() for x in (k, v))
+    vf = torch.where(torch.isfinite(vf), vf, torch.zeros_like(vf))
     s = torch.matmul(qf, kf.transpose(1, 2).contiguous()) / 16.0
     hidden = torch.arange(n, device="cuda")[None] > past + torch.arange(T, device="cuda")[:, None]
     s = s.masked_fill(hidden, float("-inf"))
@@ -77,6 +81,37 @@ def test_streaming_forms_rescale(gpu, direction, T, past):
     assert_bf16_close(out, expect, what=f"ramp {direction} T={T} past={past}")
 
 
+# A V row with an infinity or a NaN reaches exactly the tokens that see its key, as in a scalar sum: a masked key has
+# probability 0, and 0 times such a value must not count.  Hit are a past row (if there is one), the first and the
+# last new token, two neighbours inside a query tile and one in a later key tile of it, each in a dim of its own.
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("T,past,layout", [(600, 1020, 0), (600, 1020, 1), (1030, 0, 1), (1041, 0, 0), (1041, 30, 1),
+                                           (2049, 0, 1), (2049, 0, 0), (2081, 40, 1)])
+def test_streaming_forms_non_finite_values_reach_only_their_readers(gpu, T, past, layout, value):
+    def readers(hits):  # first new token that sees each hit (dim, past + token)
+        first = torch.full((D,), T, device="cuda")
+        for d, row in hits:
+            first[d] = max(0, row - past)
+        return torch.arange(T, device="cuda")[:, None] >= first[None]  # [T][D]
+
+    tokens = sorted({0, 8, 9, 17, 30, T - 1} & set(range(T)))
+    hits = [(3 + 31 * i, past + t) for i, t in enumerate(tokens)] + ([(250, past - 1)] if past else [])
+
+    def edit(k, v):
+        for d, row in hits:
+            v[row, 1, d] = value
+
+    out, ref, same = attend(T, past, layout, seed=T + past, edit=edit)
+    seen = torch.zeros(T, HQ, D, dtype=torch.bool, device="cuda")
+    seen[:, 4:8] = readers(hits)[:, None]  # query heads of KV head 1
+    got = out.float()
+    assert torch.isnan(got[seen]).all() if value != value else (got[seen] == value).all()
+    clean = torch.where(seen, torch.zeros_like(got), got)
+    assert torch.isfinite(clean).all(), "a token that does not see the key"
+    want = torch.where(seen, torch.zeros_like(ref), ref)
+    assert_bf16_close(from_dev(clean), from_dev(want), what=f"prefill T={T} past={past} layout={layout}")
+
+
 @pytest.mark.parametrize("T,past,rot,wdt,layout", [(17, 1011, 64, torch.bfloat16, 1), (100, 1000, 8, torch.float32, 0),
                                                    (520, 600, 256, torch.float32, 1), (1030, 0, 64, torch.bfloat16, 1),
                                                    (2050, 3, 192, torch.bfloat16, 0), (2079, 0, 256, torch.float32, 1)])
@@ -84,6 +119,21 @@ def test_streaming_forms_fused_equal_producers_then_attention(gpu, T, past, rot,
     c = _prefill_case(T, past, rot, wdt, layout, seed=T + past)
     assert torch.equal(c["cache1"], c["cache2"])
     assert torch.equal(c["out1"], c["out2"])
+
+
+@pytest.mark.parametrize("T,past,rot,wdt,layout", [(521, 1000, 64, torch.bfloat16, 1), (1030, 0, 8, torch.float32, 0),
+                                                   (2049, 3, 256, torch.float32, 1), (2080, 0, 24, torch.bfloat16, 0)])
+def test_streaming_forms_fused_non_finite_values(gpu, T, past, rot, wdt, layout):
+    # The same call with infinite values in a few tokens (the unfused one is compared with torch above).
+    def edit(v):
+        for t in (9, 300, 301, T - 1):
+            v[t, 2, t % D] = np.inf
+
+    c = _prefill_case(T, past, rot, wdt, layout, seed=T, edit_v=edit)
+    out1, out2 = (c[x].view(T, HQ, D) for x in ("out1", "out2"))
+    assert torch.isinf(out2[9:, 8:12, 9]).all() and torch.isfinite(out2[:9]).all()
+    assert torch.isinf(out2).sum() == 4 * sum(T - t for t in (9, 300, 301, T - 1)) and not torch.isnan(out2).any()
+    assert torch.equal(out1, out2) and torch.equal(c["cache1"], c["cache2"])
 
 
 # ---- the f32 cache at the model shape (K, V and the probabilities at f32 precision; tiles of 16 keys, a round of 64)
