@@ -356,6 +356,8 @@ void launch_prefill(const void *q, const void *k, const void *v, const void *g, 
     const auto bits = [](const void *p) { return reinterpret_cast<std::uintptr_t>(p); };
     mfma = ((bits(q) | bits(cache)) & 15u) == 0 && ((bits(g) | bits(o)) & 7u) == 0 &&
            s.query_heads == kQueryHeads && s.kv_heads == kKvHeads && s.head_dim == kHeadDim;
+    // (the kernel of the f32 cache loads the gate by 16-byte LDS-direct loads)
+    if constexpr (!std::is_same_v<CacheT, bf16_bits>) mfma = mfma && (bits(g) & 15u) == 0;
     // A prompt with no past reads its keys straight from key/value and
     // appends them inside the attention kernel.
     fused = mfma && std::is_same_v<CacheT, bf16_bits> && s.past_tokens == 0 && ((bits(k) | bits(v)) & 15u) == 0;

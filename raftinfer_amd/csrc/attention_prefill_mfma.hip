@@ -560,7 +560,10 @@ void launch_prefill_mfma(const bf16_bits *q, const bf16_bits *key, const bf16_bi
                          const bf16_bits *gate, bf16_bits *out, bf16_bits *cache,
                          std::size_t tokens, std::size_t max_ctx, std::size_t past,
                          bool head_major, bool fused_append, hipStream_t stream) {
-  const PrefillForm form = prefill_plan(tokens, past);
+  // The streaming forms bring the gate rows by 16-byte LDS-direct loads; a gate
+  // that is only 8-byte aligned stays with the vector loads of the short form.
+  const bool gate_aligned = (reinterpret_cast<std::uintptr_t>(gate) & 15u) == 0;
+  const PrefillForm form = gate_aligned ? prefill_plan(tokens, past) : PrefillForm::short8;
   if (form != PrefillForm::short8) {
     launch_prefill_wide(form, q, key, value, gate, out, cache, tokens, max_ctx, past, head_major, fused_append, nullptr,
                         stream);

@@ -17,7 +17,7 @@ void launch_prefill_mfma(const bf16_bits *q, const bf16_bits *key, const bf16_bi
                          bool head_major, bool fused_append, hipStream_t stream);
 
 // The same with an f32 cache, used at full precision; the cache must already hold
-// positions 0..past+tokens-1.
+// positions 0..past+tokens-1, and gate is 16-byte aligned.
 void launch_prefill_f32_cache(const bf16_bits *q, const bf16_bits *gate, bf16_bits *out,
                               float *cache, std::size_t tokens, std::size_t max_ctx,
                               std::size_t past, bool head_major, hipStream_t stream);
@@ -46,7 +46,7 @@ PrefillForm prefill_plan(std::size_t tokens, std::size_t past);
 namespace prefill {
 struct PrefillNormRope;
 }
-// The streaming forms; the same requirements.  With nq != nullptr q is the raw q
+// The streaming forms; the same requirements, and gate 16-byte aligned.  With nq != nullptr q is the raw q
 // projection (gate, key and value are not read) and the cache holds every key.
 void launch_prefill_wide(PrefillForm form, const bf16_bits *q, const bf16_bits *key,
                          const bf16_bits *value, const bf16_bits *gate, bf16_bits *out,

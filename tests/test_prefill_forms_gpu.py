@@ -13,9 +13,15 @@ from test_fused_gpu import _prefill_case
 pytestmark = pytest.mark.gpu
 
 
-def attend(T, past, layout, seed, edit=None):
+def shifted(t, elements=4):
+    """A copy of t that starts `elements` past an allocation (8 bytes for the default of 4 bf16 values)."""
+    flat = torch.empty(t.numel() + elements, device=t.device, dtype=t.dtype)[elements:]
+    return flat.copy_(t.flatten()).view(t.shape)
+
+
+def attend(T, past, layout, seed, edit=None, place=lambda t: t):
     """Output, torch fp32 reference (non-finite values of V taken as 0) and whether the cache was written as expected,
-    for random inputs; edit(k, v) changes the rows [past + T][4][256] before the call."""
+    for random inputs; edit(k, v) changes the rows [past + T][4][256] before the call, place puts gate and output."""
     g = torch.Generator(device="cuda").manual_seed(seed)
     rnd = lambda *shape: torch.randn(*shape, device="cuda", generator=g).to(torch.bfloat16)
     n = past + T
@@ -26,7 +32,7 @@ def attend(T, past, layout, seed, edit=None):
     full = rows.clone()
     rows[:, past:] = 0
     cache = (rows.transpose(1, 2) if layout == 1 else rows).contiguous()
-    out = torch.empty(T, HQ, D, device="cuda", dtype=torch.bfloat16)
+    gate, out = place(gate), place(torch.empty(T, HQ, D, device="cuda", dtype=torch.bfloat16))
     ops.qwen35_causal_attention(q, k[past:].contiguous(), v[past:].contiguous(), gate, out, cache, None,
                                 S(T, HQ, HKV, D, n, past), 3, ops.Qwen35AttentionLaunchPolicy(1, 1, layout))
     torch.cuda.synchronize()
@@ -136,8 +142,17 @@ def test_streaming_forms_fused_non_finite_values(gpu, T, past, rot, wdt, layout)
     assert torch.equal(out1, out2) and torch.equal(c["cache1"], c["cache2"])
 
 
+# Gate and output are accepted at 8-byte alignment, at sizes where each streaming form would take an aligned call.
+@pytest.mark.parametrize("T,past,layout", [(10, 1020, 1), (600, 1020, 0), (1030, 0, 1), (2049, 0, 1)])
+def test_gate_and_output_at_8_byte_alignment(gpu, T, past, layout):
+    out, ref, same = attend(T, past, layout, seed=T, place=shifted)
+    assert out.data_ptr() % 16 == 8
+    assert same, "appended rows"
+    assert_bf16_close(from_dev(out), from_dev(ref), what=f"prefill T={T} past={past} layout={layout}")
+
+
 # ---- the f32 cache at the model shape (K, V and the probabilities at f32 precision; tiles of 16 keys, a round of 64)
-def f32_cache(T, past, layout, seed, exact_bf16=False, edit=None):
+def f32_cache(T, past, layout, seed, exact_bf16=False, edit=None, place=lambda t: t):
     g = torch.Generator(device="cuda").manual_seed(seed)
     rnd = lambda *shape: torch.randn(*shape, device="cuda", generator=g)
     n = past + T
@@ -151,7 +166,7 @@ def f32_cache(T, past, layout, seed, exact_bf16=False, edit=None):
     cache = rows.clone()
     cache[:, past:] = 0
     cache = (cache.transpose(1, 2) if layout == 1 else cache).contiguous()
-    out = torch.empty(T, HQ, D, device="cuda", dtype=torch.bfloat16)
+    gate, out = place(gate), place(torch.empty(T, HQ, D, device="cuda", dtype=torch.bfloat16))
     ops.qwen35_causal_attention(q, rows[0, past:].bfloat16(), rows[1, past:].bfloat16(), gate, out, cache, None,
                                 S(T, HQ, HKV, D, n, past), 3, ops.Qwen35AttentionLaunchPolicy(1, 0, layout))
     torch.cuda.synchronize()
@@ -172,6 +187,13 @@ def test_f32_cache_prefill(gpu, T, past, layout, exact_bf16):
     got = from_dev(out)
     # f32 sums of about 1e-6 of the largest product each, then one rounding to bf16 (2^-8 of the value at most)
     assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) * 1.001 + 2e-5)
+
+
+def test_f32_cache_prefill_gate_and_output_at_8_byte_alignment(gpu):
+    out, p, v, gate, _, same = f32_cache(65, 70, 1, seed=8, place=shifted)
+    assert same and out.data_ptr() % 16 == 8
+    want = (torch.matmul(p, v).permute(1, 0, 2) * torch.sigmoid(gate)).cpu().numpy()
+    assert np.all(np.abs(from_dev(out) - want) <= 2.0 ** -8 * np.abs(want) * 1.001 + 2e-5)
 
 
 def test_f32_cache_prefill_keeps_bits_below_bf16(gpu):
