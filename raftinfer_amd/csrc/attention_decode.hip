@@ -654,7 +654,8 @@ __device__ __forceinline__ void scan_split_body(unsigned block, const ScanArgs<A
                                                 float *__restrict__ pmax, float *__restrict__ psum,
                                                 float *__restrict__ pval, std::size_t position,
                                                 std::size_t capacity, std::size_t max_partitions,
-                                                std::size_t partition_tokens, ScanShared<DS, kScanWaves> &sh) {
+                                                std::size_t partition_tokens, bool append,
+                                                ScanShared<DS, kScanWaves> &sh) {
   constexpr int kDims = kHeadDim / DS;
   const std::size_t ctx = position + 1;
   std::size_t unit;
@@ -666,12 +667,14 @@ __device__ __forceinline__ void scan_split_body(unsigned block, const ScanArgs<A
   const std::size_t begin = partition * partition_tokens;
   if (begin >= ctx) return;
   const std::size_t end = ctx < begin + partition_tokens ? ctx : begin + partition_tokens;
-  scan_slice<ActT, CacheT, DS, kScanWaves, scan_unroll(DS)>(a, kv_head, dq, begin, end, position, sh);
+  // (without the append the new token's row is the cache's, and its inputs are not read)
+  scan_slice<ActT, CacheT, DS, kScanWaves, scan_unroll(DS)>(a, kv_head, dq, begin, end,
+                                                            append ? position : ~std::size_t{0}, sh);
   __syncthreads();
   // the append, also of a position past the plan's capacity (see split_body)
   const bool owns_position = position >= begin && position < end;
   const bool past_capacity = partition + 1 == capacity && position >= begin + partition_tokens;
-  if (dq == 0 && (owns_position || past_capacity)) append_rows(a, kv_head, position);
+  if (append && dq == 0 && (owns_position || past_capacity)) append_rows(a, kv_head, position);
   for (int o = threadIdx.x; o < kGroup * kDims; o += kScanWaves * 64) {
     const int h = o / kDims, d = o % kDims;
     float mm, l, acc;
@@ -711,7 +714,7 @@ __global__ __launch_bounds__(kScanWaves * 64) void decode_scan_kernel(
   if (position >= a.max_ctx) return;
   if (position + 1 >= threshold)
     scan_split_body<ActT, CacheT, DS>(blockIdx.x, a, pmax, psum, pval, position, capacity, max_partitions,
-                                      partition_tokens, sh.split);
+                                      partition_tokens, !partition_only, sh.split);
   else if (!partition_only)
     scan_single_body(blockIdx.x, a, gate, output, position, sh.single);
 }

@@ -562,3 +562,39 @@ def test_scan_decode_slices(gpu, act, cdt, layout, ctx, max_ctx, mode):
         assert close_enough(out, expect), (device_position,)
         ck, cv = read_cache(cache, layout, ctx, max_ctx)
         assert np.array_equal(ck, keys) and np.array_equal(cv, vals)
+
+
+@pytest.mark.parametrize("act,cdt,ctx,max_ctx", [(3, 0, 600, 1024), (1, 1, 777, 1024), (1, 0, 6400, 6400)])
+def test_partition_only_reads_the_cache_and_leaves_it(gpu, act, cdt, ctx, max_ctx):
+    # The measurement entry enqueues the partition kernel alone: it scans the rows that the cache holds, the new token's
+    # among them, and appends nothing (the bf16 / bf16 kernel, which forms the append too, is not meant here).
+    import ctypes
+
+    from raftinfer_amd import _lib
+    r = rng(ctx)
+    keys, vals, q = normal(r, ctx, HKV, D), normal(r, ctx, HKV, D), normal(r, HQ, D)
+    if cdt == 1:
+        keys, vals = bf16(keys), bf16(vals)
+    q = bf16(q) if act == 3 else q
+    cache = to_dev(make_cache(keys, vals, 0, max_ctx), CDT[cdt])
+    before = cache.clone()
+    qd = to_dev(q, TDT[act])
+    junk = torch.full((HKV * D,), float("nan"), device="cuda", dtype=TDT[act])
+    out = torch.empty(HQ * D, device="cuda", dtype=TDT[act])
+    shape = S(1, HQ, HKV, D, max_ctx, ctx - 1)
+    plan = ops.qwen35_online_decode_plan(shape, ops.SPLIT_K_256, ctx)
+    count, max_at, sum_at, value_at, nbytes = ops.qwen35_online_decode_workspace_layout(shape, plan[0])
+    ws = torch.empty(nbytes, device="cuda", dtype=torch.uint8)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    stream = ops._stream(None)
+    _lib.check(_lib.load().raftinfer_amd_online_attention_decode_partition_only(
+        ptr(qd), ptr(junk), ptr(junk), ptr(qd), ptr(out), ptr(cache), cache.numel() * cache.element_size(), ptr(ws),
+        nbytes, shape.c(), act, cdt, 0, _lib.DecodePlan(*plan), None, stream))
+    torch.cuda.synchronize()
+    assert torch.equal(cache, before)
+    parts, active = -(-max_ctx // 256), -(-ctx // 256)
+    f = ws.cpu().numpy().view(np.float32)
+    em, es, ev = orc.decode_partials(q, keys, vals, ctx, 256, parts)
+    for at, want in ((max_at, em), (sum_at, es), (value_at, ev)):
+        got = f[at // 4:at // 4 + want.size].reshape(HQ, parts, -1)[:, :active]
+        assert close_enough(got, want.reshape(HQ, parts, -1)[:, :active])
