@@ -614,38 +614,48 @@ __global__ __launch_bounds__(WAVES * 64) void decode_dynamic_mfma_kernel(
                                       max_partitions, partition_tokens, f, psh, fq);
 }
 
-// ---- f32 activations or f32 caches (scan_slice).  The same split of the work
-// as the bf16 kernels: a workgroup per (KV head, partition, dims slice), the
-// slices of a partition on one XCD, each computing the scores of all its keys and
-// reading its own part of V.  With the whole 256 dims in one workgroup a context
-// of 3000 tokens had 48 workgroups, and a step was four launches (append, early
-// exit of the single-block kernel, partitions, merge): 26.5 us on an f32
-// token-major cache, 15 of them the partitions.  Sliced, with the append and the
-// choice of path inside, it is two launches and 16.0 us, 11.4 to 12.5 of them the
-// partitions: with four slices they read 61 MB (K four times, V once; 25 MB are
-// the cache's own) and repeat the scores four times on the vector units.
+// ---- f32 activations or f32 caches (scan_slice).  A split step: a workgroup per
+// (KV head, partition, dims slice), the slices of a partition on one XCD, each
+// computing the scores of all its keys and reading its own part of V.  With the whole
+// 256 dims in one workgroup a context of 3000 tokens had 48 workgroups, and a step was
+// four launches (append, early exit of the single-block kernel, partitions, merge):
+// 26.6 us on an f32 token-major cache, 15 of them the partitions.  Sliced, with the
+// append and the choice of path inside, it is two launches and 15.9 us, 11.4 to 12.5
+// of them the partitions: with four slices they read 61 MB (K four times, V once; 25
+// MB are the cache's own) and repeat the scores four times on the vector units.
+//
+// A single-block step: a workgroup per (query head, one of four dims slices).  The
+// scores bound it, so a workgroup has those of one head: all four heads of a KV head
+// in each of sixteen slices took 8.5 us at 255 tokens and 14.9 at 700 of an f32 cache
+// (now 5.5 and 9.4), and on a bf16 cache 15.5 at 700, more than the 13.4 of one
+// workgroup per head with all dims (now 8.1).  Two tokens per row-group and step on
+// f32 rows, four on bf16 rows: 4000 bf16 tokens 39 -> 32 us, 200 f32 tokens 5.1
+// against 5.6.
 constexpr int kScanWaves = 8;
+constexpr int kScanSingleDs = 4;
+template <typename CacheT> constexpr int kScanSingleUnroll = sizeof(CacheT) == 4 ? 2 : 4;
+using ScanSingleShared = ScanShared<1, kScanSingleDs, kScanWaves>;
 constexpr int scan_unroll(int ds) { return ds == 1 ? 2 : 4; } // tokens per row-group and step (registers)
 
 template <typename ActT, typename CacheT>
 __device__ __forceinline__ void scan_single_body(unsigned block, const ScanArgs<ActT, CacheT> &a,
                                                  const ActT *__restrict__ gate, ActT *__restrict__ output,
-                                                 std::size_t position, ScanShared<kSingleDs, kScanWaves> &sh) {
-  constexpr int DS = kSingleDs, kDims = kHeadDim / DS;
-  std::size_t kv_head;
+                                                 std::size_t position, ScanSingleShared &sh) {
+  constexpr int DS = kScanSingleDs, kDims = kHeadDim / DS;
+  std::size_t head;
   int dq;
-  xcd_unit<DS>(block, kv_head, dq);
-  if (kv_head >= kKvHeads) return;
-  const int o = threadIdx.x, h = o / kDims, d = o % kDims; // the first 4 x 16 threads finish an output
-  const std::size_t idx = (kv_head * kGroup + h) * kHeadDim + dq * kDims + d;
-  const bool finisher = o < kGroup * kDims;
+  xcd_unit<DS>(block, head, dq);
+  if (head >= kQueryHeads) return;
+  const int d = threadIdx.x; // the first kDims threads finish an output each
+  const bool finisher = d < kDims;
+  const std::size_t idx = head * kHeadDim + dq * kDims + d;
   const float gv = finisher ? Elem<ActT>::load(gate, idx) : 0.f;
-  scan_slice<ActT, CacheT, DS, kScanWaves, scan_unroll(DS)>(a, kv_head, dq, 0, position + 1, position, sh);
+  scan_slice<ActT, CacheT, 1, DS, kScanWaves, kScanSingleUnroll<CacheT>>(a, head, dq, 0, position + 1, position, sh);
   __syncthreads();
-  if (dq == 0) append_rows(a, kv_head, position);
+  if (dq == 0 && head % kGroup == 0) append_rows(a, head / kGroup, position);
   if (!finisher) return;
   float mm, l, acc;
-  combine_waves(sh, h, d, mm, l, acc);
+  combine_waves(sh, 0, d, mm, l, acc);
   Elem<ActT>::store(output, idx, (acc / l) * sigmoid_gate(gv));
 }
 
@@ -655,21 +665,25 @@ __device__ __forceinline__ void scan_split_body(unsigned block, const ScanArgs<A
                                                 float *__restrict__ pval, std::size_t position,
                                                 std::size_t capacity, std::size_t max_partitions,
                                                 std::size_t partition_tokens, bool append,
-                                                ScanShared<DS, kScanWaves> &sh) {
+                                                ScanShared<kGroup, DS, kScanWaves> &sh) {
   constexpr int kDims = kHeadDim / DS;
   const std::size_t ctx = position + 1;
   std::size_t unit;
   int dq;
   xcd_unit<DS>(block, unit, dq);
   if (unit >= kKvHeads * capacity) return;
-  const std::size_t kv_head = DS == 1 ? unit % kKvHeads : unit / capacity;
-  const std::size_t partition = DS == 1 ? unit / kKvHeads : unit % capacity;
+  // The four KV heads of a partition run side by side where their f32 rows lie side by
+  // side (token-major, 32768 tokens from memory: 69 -> 62 us); rows of one head follow
+  // each other otherwise (head-major f32 67 -> 57 us, bf16 42 -> 39.5).
+  const bool heads_first = DS == 1 && sizeof(CacheT) == 4 && !a.head_major;
+  const std::size_t kv_head = heads_first ? unit % kKvHeads : unit / capacity;
+  const std::size_t partition = heads_first ? unit / kKvHeads : unit % capacity;
   const std::size_t begin = partition * partition_tokens;
   if (begin >= ctx) return;
   const std::size_t end = ctx < begin + partition_tokens ? ctx : begin + partition_tokens;
   // (without the append the new token's row is the cache's, and its inputs are not read)
-  scan_slice<ActT, CacheT, DS, kScanWaves, scan_unroll(DS)>(a, kv_head, dq, begin, end,
-                                                            append ? position : ~std::size_t{0}, sh);
+  scan_slice<ActT, CacheT, kGroup, DS, kScanWaves, scan_unroll(DS)>(a, kv_head * kGroup, dq, begin, end,
+                                                                    append ? position : ~std::size_t{0}, sh);
   __syncthreads();
   // the append, also of a position past the plan's capacity (see split_body)
   const bool owns_position = position >= begin && position < end;
@@ -692,7 +706,7 @@ template <typename ActT, typename CacheT>
 __global__ __launch_bounds__(kScanWaves * 64) void decode_scan_single_kernel(
     ScanArgs<ActT, CacheT> a, const ActT *__restrict__ gate, ActT *__restrict__ output, std::size_t host_position,
     const std::uint32_t *device_position) {
-  __shared__ ScanShared<kSingleDs, kScanWaves> sh;
+  __shared__ ScanSingleShared sh;
   const std::size_t position = read_position(device_position, host_position);
   if (position >= a.max_ctx) return;
   scan_single_body(blockIdx.x, a, gate, output, position, sh);
@@ -707,8 +721,8 @@ __global__ __launch_bounds__(kScanWaves * 64) void decode_scan_kernel(
     const std::uint32_t *device_position, std::size_t capacity, std::size_t max_partitions,
     std::size_t partition_tokens, std::size_t threshold, bool partition_only) {
   __shared__ union Shared {
-    ScanShared<kSingleDs, kScanWaves> single;
-    ScanShared<DS, kScanWaves> split;
+    ScanSingleShared single;
+    ScanShared<kGroup, DS, kScanWaves> split;
   } sh;
   const std::size_t position = read_position(device_position, host_position);
   if (position >= a.max_ctx) return;
@@ -882,7 +896,7 @@ void launch_decode(const void *query, const void *key, const void *value, const 
   if (partition_only) require<Err>(plan.partition_tokens != 0, "partition-only decode needs a split-K plan");
   const ScanArgs<ActT, CacheT> args{q, static_cast<const ActT *>(key), static_cast<const ActT *>(value), cache,
                                     shape.max_context_tokens, head_major};
-  const unsigned single_grid = xcd_grid<kSingleDs>(kKvHeads);
+  const unsigned single_grid = xcd_grid<kScanSingleDs>(kQueryHeads);
   const std::size_t host_ctx = shape.past_tokens + 1;
   if (single || (device_position == nullptr && !partition_only && host_ctx < plan.split_k_threshold_tokens)) {
     decode_scan_single_kernel<ActT, CacheT><<<single_grid, kScanWaves * 64, 0, stream>>>(
@@ -1234,7 +1248,7 @@ __global__ __launch_bounds__(WAVES * 64) void batched_partition_kernel(
     std::size_t cache_stride, std::size_t max_ctx, const std::uint32_t *__restrict__ lengths,
     std::size_t max_partitions, std::size_t single_max, float *__restrict__ pmax,
     float *__restrict__ psum, float *__restrict__ pval) {
-  __shared__ ScanShared<1, WAVES> sh;
+  __shared__ ScanShared<kGroup, 1, WAVES> sh;
   const std::size_t seq = blockIdx.y;
   const std::size_t unit = blockIdx.x / max_partitions;
   const std::size_t partition = blockIdx.x % max_partitions;
@@ -1247,7 +1261,7 @@ __global__ __launch_bounds__(WAVES * 64) void batched_partition_kernel(
   const ScanArgs<ActT, bf16_bits> a{query + seq * kQueryHeads * kHeadDim, key + seq * kKvHeads * kHeadDim,
                                     value + seq * kKvHeads * kHeadDim,
                                     reinterpret_cast<bf16_bits *>(cache_base + seq * cache_stride), max_ctx, true};
-  scan_slice<ActT, bf16_bits, 1, WAVES, U>(a, unit, 0, begin, end, ctx - 1, sh);
+  scan_slice<ActT, bf16_bits, kGroup, 1, WAVES, U>(a, unit * kGroup, 0, begin, end, ctx - 1, sh);
   __syncthreads();
   if (ctx - 1 >= begin && ctx - 1 < end) append_rows(a, unit, ctx - 1);
   for (int o = threadIdx.x; o < kGroup * kHeadDim; o += WAVES * 64) {

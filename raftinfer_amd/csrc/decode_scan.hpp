@@ -1,11 +1,12 @@
 // Device core of the decode kernels for f32 activations or f32 caches (the
 // bf16 / bf16 kernels have theirs in decode_mfma.hpp): one workgroup scans a
-// token range of one KV head for the four query heads of its GQA group and one
-// slice of the output dims, keeping an online-softmax state per head.
+// token range of one KV head for one or all four query heads of its GQA group and
+// one slice of the output dims, keeping an online-softmax state per head.
 //
 // Lane layout (wave64 = 4 row-groups of 16 lanes): row-group g takes one token
 // per step, and a row is read in 16-byte pieces, 16 lanes on one contiguous
-// 256-byte stretch (whole 128-byte lines).  q.k partial dots reduce inside the
+// 256-byte stretch (whole 128-byte lines; a bf16 V slice of 64 dims in 8-byte
+// pieces, one line).  q.k partial dots reduce inside the
 // 16-lane row with four DPP steps; the softmax runs in the exp2 domain with
 // log2(e)/sqrt(D) folded into q.
 #pragma once
@@ -29,16 +30,15 @@ __device__ __forceinline__ std::size_t cache_row(bool head_major, std::size_t to
                     : (token * kKvHeads + kv_head) * kHeadDim;
 }
 
-// W contiguous cache elements as loaded (kOnce: read by one workgroup only, so
-// streamed past the caches).
-template <typename T, int W, bool kOnce> struct Piece {
+// W contiguous cache elements as loaded (kStream: nontemporal).
+template <typename T, int W, bool kStream> struct Piece {
   static_assert(W * sizeof(T) <= 16);
   typedef T vec __attribute__((ext_vector_type(W == 1 ? 2 : W)));
   using Raw = std::conditional_t<W == 1, T, vec>;
   Raw raw;
   __device__ __forceinline__ void load(const T *p) {
     const auto *v = reinterpret_cast<const Raw *>(p);
-    if constexpr (kOnce) raw = __builtin_nontemporal_load(v); else raw = *v;
+    if constexpr (kStream) raw = __builtin_nontemporal_load(v); else raw = *v;
   }
   __device__ __forceinline__ void set(int i, T x) {
     if constexpr (W == 1) raw = x; else raw[i] = x;
@@ -60,21 +60,23 @@ template <typename ActT, typename CacheT> struct ScanArgs {
 };
 
 // Per-head combined state after a workgroup scan, staged in LDS.
-template <int DS, int WAVES> struct ScanShared {
-  float m[WAVES][kGroup];
-  float l[WAVES][kGroup];
-  float acc[WAVES][kGroup][kHeadDim / DS];
+template <int NH, int DS, int WAVES> struct ScanShared {
+  float m[WAVES][NH];
+  float l[WAVES][NH];
+  float acc[WAVES][NH][kHeadDim / DS];
 };
 
-// Scans tokens [begin, end) of kv_head, dims slice dq of 256 / DS for the
-// output, and leaves the per-wave states in `sh`.  The row of position `pos` (if
+// Scans tokens [begin, end) for the query heads head .. head + NH - 1 of one KV
+// head, dims slice dq of 256 / DS for the output, and leaves the per-wave states in `sh`.  The row of position `pos` (if
 // in range) comes from key_new / value_new, as the cache stores it.  U tokens per
 // row-group and step.  Every wave returns after writing its slot; the caller
 // synchronizes.
-template <typename ActT, typename CacheT, int DS, int WAVES, int U>
-__device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std::size_t kv_head, int dq,
+template <typename ActT, typename CacheT, int NH, int DS, int WAVES, int U>
+__device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std::size_t head, int dq,
                                            std::size_t begin, std::size_t end, std::size_t pos,
-                                           ScanShared<DS, WAVES> &sh) {
+                                           ScanShared<NH, DS, WAVES> &sh) {
+  static_assert(kGroup % NH == 0, "the heads of one KV head");
+  const std::size_t kv_head = head / kGroup;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int g = lane >> 4;
@@ -83,22 +85,29 @@ __device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std:
   constexpr int kDims = kHeadDim / DS, kPerLane = kDims / 16; // output dims of the slice, of a lane
   constexpr int KW = 16 / sizeof(CacheT), KP = 16 / KW;       // K piece width, pieces per lane
   constexpr int VW = kPerLane < KW ? kPerLane : KW, VP = kPerLane / VW;
+  // Which rows are streamed past the caches.  One dims slice reads a row once; with
+  // both K and V streamed a cache of 134 MB (32768 tokens, one layer over and over)
+  // took 61 us where K alone takes 55, and with neither a cache that has to come from
+  // memory 65 where K alone takes 62.  Slices share K.  Their V rows are their own,
+  // but only two f32 slices gain from streaming (8000 tokens from memory: 23.0 -> 20.5
+  // us; four f32 slices at 3000 tokens 14.3 -> 15.8, bf16 rows 15.3 -> 15.8 at 6000).
+  constexpr bool kStreamK = DS == 1, kStreamV = DS == 2 && sizeof(CacheT) == 4;
   // Element of piece p of a lane: 16 KW p + KW r (K), 16 VW p + VW r of the slice (V).
   const CacheT *k_plane = a.cache + cache_row(a.head_major, 0, kv_head, a.max_ctx);
   const CacheT *v_plane = k_plane + a.max_ctx * kKvHeads * kHeadDim + dq * kDims;
   const std::size_t token_stride = a.head_major ? kHeadDim : kKvHeads * kHeadDim;
 
-  float q[kGroup][16];
+  float q[NH][16];
 #pragma unroll
-  for (int h = 0; h < kGroup; ++h) {
-    const ActT *qh = a.query + (kv_head * kGroup + h) * kHeadDim;
+  for (int h = 0; h < NH; ++h) {
+    const ActT *qh = a.query + (head + h) * kHeadDim;
 #pragma unroll
     for (int i = 0; i < 16; ++i) q[h][i] = Elem<ActT>::load(qh, 16 * KW * (i / KW) + KW * r + i % KW) * qscale;
   }
 
-  float m[kGroup], l[kGroup], acc[kGroup][kPerLane];
+  float m[NH], l[NH], acc[NH][kPerLane];
 #pragma unroll
-  for (int h = 0; h < kGroup; ++h) {
+  for (int h = 0; h < NH; ++h) {
     m[h] = -INFINITY;
     l[h] = 0.f;
 #pragma unroll
@@ -108,8 +117,8 @@ __device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std:
   constexpr int kTile = 4 * U; // tokens per wave step
   for (std::size_t tile = begin + static_cast<std::size_t>(wave) * kTile; tile < end;
        tile += static_cast<std::size_t>(WAVES) * kTile) {
-    Piece<CacheT, KW, DS == 1> k[U][KP];
-    Piece<CacheT, VW, true> v[U][VP];
+    Piece<CacheT, KW, kStreamK> k[U][KP];
+    Piece<CacheT, VW, kStreamV> v[U][VP];
     const bool whole = tile + kTile <= end; // (uniform)
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -139,11 +148,11 @@ __device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std:
         }
       }
     }
-    float s[kGroup][U];
+    float s[NH][U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
 #pragma unroll
-      for (int h = 0; h < kGroup; ++h) {
+      for (int h = 0; h < NH; ++h) {
         float d0 = 0.f, d1 = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -160,13 +169,13 @@ __device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std:
       for (int u = 0; u < U; ++u) {
         if (tile + 4 * u + g < end) continue;
 #pragma unroll
-        for (int h = 0; h < kGroup; ++h) s[h][u] = -INFINITY;
+        for (int h = 0; h < NH; ++h) s[h][u] = -INFINITY;
 #pragma unroll
         for (int i = 0; i < kPerLane; ++i) v[u][i / VW].set(i % VW, CacheT{});
       }
     }
 #pragma unroll
-    for (int h = 0; h < kGroup; ++h) {
+    for (int h = 0; h < NH; ++h) {
       float mt = m[h];
 #pragma unroll
       for (int u = 0; u < U; ++u) mt = fmaxf(mt, s[h][u]);
@@ -194,7 +203,7 @@ __device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std:
   // Combine the four row-groups of the wave (lanes r, r^16, r^32, r^48 own
   // the same dims).
 #pragma unroll
-  for (int h = 0; h < kGroup; ++h) {
+  for (int h = 0; h < NH; ++h) {
     float mm = fmaxf(m[h], xor16(m[h]));
     mm = fmaxf(mm, xor32(mm));
     const float w = m[h] == -INFINITY ? 0.f : exp2f(m[h] - mm);
@@ -221,8 +230,8 @@ __device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std:
 
 // Merges the per-wave states of `sh` for output element (h, d of the slice):
 // returns the exp2-domain max, the sum and the unnormalised accumulator.
-template <int DS, int WAVES>
-__device__ __forceinline__ void combine_waves(const ScanShared<DS, WAVES> &sh, int h, int d,
+template <int NH, int DS, int WAVES>
+__device__ __forceinline__ void combine_waves(const ScanShared<NH, DS, WAVES> &sh, int h, int d,
                                               float &m_out, float &l_out, float &a_out) {
   float mm = -INFINITY;
 #pragma unroll
