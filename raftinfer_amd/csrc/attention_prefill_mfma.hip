@@ -543,17 +543,27 @@ __global__ __launch_bounds__(kThreads) void prefill_mfma_kernel(
 // So the lines lie where the workgroups of a form come to 256 (512, 1024, 2048
 // tokens), and below them where the longer start and end of the streaming
 // kernel is made up for.  Measured (us; short8 / stream8 / stream16 / stream32,
-// tokens behind past keys): 512 behind 0: 12.9 / 15.4 / 21 / 30, behind 512:
-// 23.5 / 23.2 / 32 / 44, behind 1024: 29.8 / 28.0 / 38 / 55; 64 behind 1024:
-// 21.2 / 19.5 / 28 / 44; 768 behind 0: 18.6 / 22 / 26 / 37, behind 1000: 49 /
-// 46 / 43 / 63; 1100 behind 0: 33 / 35 / 30 / 46; 2048 behind 0: 77 / 79 / 60 /
-// 69, behind 4000: 296 / 249 / 186 / 184; 2560 behind 0: 124 / 105 / 92 / 83;
-// 5000 behind 4000: 829 / 720 / 549 / 525.
+// tokens behind past keys):
+//   to 512, line at 1024 keys: 64 behind 600: 17.0 / 18.5 / 28, behind 1024: 21.7 /
+//     19.9 / 30 / 45; 512 behind 0: 12.9 / 15.4 / 21 / 30, behind 400: 21.9 / 22.6 /
+//     32, behind 512: 22.2 / 22.7, behind 513: 23.2 / 22.6 / 33, behind 1000: 28.0 /
+//     27.2 / 39
+//   to 1024, line at 1440: 513 behind 800: 34.7 / 33.9 / 35.7, behind 1000: 39.2 /
+//     38.5 / 38.7; 600 behind 513: 30.9 / 32.5 / 33.8, behind 1000: 41.6 / 41.1 /
+//     39.2; 900 behind 513: 40.4 / 41.4 / 41.8, behind 600: 42.1 / 41.7 / 41.6;
+//     1024 behind 513: 44.2 / 44.4 / 42.8, behind 4000: 125 / 113 / 94
+//   1024: 1025 behind 0: 29.5 / 31.4 / 29.5 / 45, 1100 behind 0: 32.1 / 33.7 / 29.9
+//   2048 and 2176: 2048 behind 0: 70 / 71 / 59.1 / 69.1, behind 2000: 171 / 157 /
+//     126.8 / 129.4; 2049 behind 0 (its 260 workgroups of 32 begin a second pass,
+//     as the 516 of 16 do): 75 / 75 / 68.2 / 69.1, behind 1000: 139 / 130 / 120 /
+//     110; 2176 behind 0: 80 / 80 / 68.7 / 71.0, 2240: 84 / 84 / 77.1 / 74.0
+//   beyond: 4096 behind 0: 228 / 218 / 172 / 148, 2304 behind 4000: 325 / 286 / 247 /
+//     256, 2500 behind 4000: 338 / 300 / 258 / 262.
 PrefillForm prefill_plan(std::size_t tokens, std::size_t past) {
-  if (tokens > 2048) return PrefillForm::stream32;
+  if (tokens > 2048 && past + tokens > 2176) return PrefillForm::stream32;
   if (tokens > 1024) return PrefillForm::stream16;
-  if (tokens > 512) return past > 512 ? PrefillForm::stream16 : PrefillForm::short8;
-  return past + tokens >= 1024 ? PrefillForm::stream8 : PrefillForm::short8;
+  if (tokens > 512) return past + tokens >= 1440 ? PrefillForm::stream16 : PrefillForm::short8;
+  return past + tokens > 1024 ? PrefillForm::stream8 : PrefillForm::short8;
 }
 
 void launch_prefill_mfma(const bf16_bits *q, const bf16_bits *key, const bf16_bits *value,

@@ -19,15 +19,18 @@ def shifted(t, elements=4):
     return flat.copy_(t.flatten()).view(t.shape)
 
 
-def attend(T, past, layout, seed, edit=None, place=lambda t: t):
+def attend(T, past, layout, seed, edit=None, place=lambda t: t, edit_all=None):
     """Output, torch fp32 reference (non-finite values of V taken as 0) and whether the cache was written as expected,
-    for random inputs; edit(k, v) changes the rows [past + T][4][256] before the call, place puts gate and output."""
+    for random inputs; edit(k, v) or edit_all(q, k, v) changes the rows [past + T][4][256] (and q)
+    before the call, place puts gate and output."""
     g = torch.Generator(device="cuda").manual_seed(seed)
     rnd = lambda *shape: torch.randn(*shape, device="cuda", generator=g).to(torch.bfloat16)
     n = past + T
     q, gate, k, v = rnd(T, HQ, D), rnd(T, HQ, D), rnd(n, HKV, D), rnd(n, HKV, D)
     if edit is not None:
         edit(k, v)
+    if edit_all is not None:
+        edit_all(q, k, v)
     rows = torch.stack([k, v])  # token-major
     full = rows.clone()
     rows[:, past:] = 0
@@ -52,7 +55,8 @@ def attend(T, past, layout, seed, edit=None, place=lambda t: t):
 # query tile and of a key tile, an odd and an even number of key tiles.
 @pytest.mark.parametrize("T,past", [(2, 1022), (7, 1050), (33, 1000), (511, 513), (512, 512), (513, 513), (577, 1055),
                                     (1025, 0), (1039, 0), (1040, 65), (1072, 31), (2049, 0), (2080, 0), (2081, 40),
-                                    (2113, 7)])
+                                    (2113, 7), (2, 1023), (512, 513), (513, 926), (513, 927), (577, 863), (1024, 416), (2176, 0), (2049, 128),
+                                    (2177, 0), (2208, 0), (2209, 40), (2241, 7)])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_streaming_forms_against_torch(gpu, T, past, layout):
     out, ref, same = attend(T, past, layout, seed=T + past)
@@ -60,7 +64,7 @@ def test_streaming_forms_against_torch(gpu, T, past, layout):
     assert_bf16_close(from_dev(out), from_dev(ref), what=f"prefill T={T} past={past} layout={layout}")
 
 
-@pytest.mark.parametrize("T,past", [(40, 1000), (700, 600)])
+@pytest.mark.parametrize("T,past", [(40, 1000), (700, 600), (540, 920)])
 def test_streaming_forms_against_oracle(gpu, T, past):
     out, expect, cache, keys, vals = run_prefill(3, 1, 1, T, HQ, HKV, D, past, seed=T)
     assert_bf16_close(out, expect, what=f"prefill T={T} past={past}")
@@ -68,11 +72,9 @@ def test_streaming_forms_against_oracle(gpu, T, past):
     assert np.array_equal(ck, keys) and np.array_equal(cv, vals)
 
 
-@pytest.mark.parametrize("direction", [1, -1])
-@pytest.mark.parametrize("T,past", [(64, 1100), (600, 520)])
-def test_streaming_forms_rescale(gpu, direction, T, past):
-    # A -80 .. +80 score ramp: ascending, the reference max moves on every tile of every wave; descending, the first
-    # keys hold all the weight.
+def score_ramp(T, past, direction):
+    """q [T][16][256] and k, v [past + T][4][256] whose scores run from -80 to +80 over the keys (or back): ascending,
+    the reference max moves on every tile of every wave; descending, the first keys hold all the weight."""
     n = past + T
     ramp = (-80.0 + 160.0 * np.arange(n) / (n - 1)) * direction
     q = np.zeros((T, HQ, D), np.float32)
@@ -82,9 +84,33 @@ def test_streaming_forms_rescale(gpu, direction, T, past):
     v = np.zeros((n, HKV, D), np.float32)
     for h in range(HKV):
         v[:, h] = 0.01 * (np.arange(n)[:, None] % 97 + np.arange(D)[None, :] + h)
+    return q, k, v
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("T,past", [(64, 1100), (600, 520), (600, 900)])
+def test_streaming_forms_rescale(gpu, direction, T, past):
+    q, k, v = score_ramp(T, past, direction)
     out, expect, *_ = run_prefill(3, 1, 1, T, HQ, HKV, D, past,
                                   inputs=(q, normal(rng(5), T, HQ, D), k[past:], v[past:], k[:past], v[:past]))
     assert_bf16_close(out, expect, what=f"ramp {direction} T={T} past={past}")
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_32_token_form_rescale(gpu, direction, layout):
+    # (torch fp32 on the bf16 inputs: the oracle takes minutes here)
+    T, past = 2200, 40
+    ramp = torch.from_numpy(score_ramp(T, past, direction)[1]).cuda()
+
+    def edit_all(q, k, v):
+        q.zero_()
+        q[:, :, 0] = 16.0
+        k.copy_(ramp)
+
+    out, ref, same = attend(T, past, layout, seed=9, edit_all=edit_all)
+    assert same, "appended rows"
+    assert_bf16_close(from_dev(out), from_dev(ref), what=f"ramp {direction} T={T} past={past} layout={layout}")
 
 
 # A V row with an infinity or a NaN reaches exactly the tokens that see its key, as in a scalar sum: a masked key has
@@ -92,7 +118,8 @@ def test_streaming_forms_rescale(gpu, direction, T, past):
 # last new token, two neighbours inside a query tile and one in a later key tile of it, each in a dim of its own.
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
 @pytest.mark.parametrize("T,past,layout", [(600, 1020, 0), (600, 1020, 1), (1030, 0, 1), (1041, 0, 0), (1041, 30, 1),
-                                           (2049, 0, 1), (2049, 0, 0), (2081, 40, 1)])
+                                           (2049, 0, 1), (2049, 0, 0), (2081, 40, 1), (2177, 0, 1), (2177, 0, 0),
+                                           (2209, 40, 1)])
 def test_streaming_forms_non_finite_values_reach_only_their_readers(gpu, T, past, layout, value):
     def readers(hits):  # first new token that sees each hit (dim, past + token)
         first = torch.full((D,), T, device="cuda")
@@ -120,7 +147,9 @@ def test_streaming_forms_non_finite_values_reach_only_their_readers(gpu, T, past
 
 @pytest.mark.parametrize("T,past,rot,wdt,layout", [(17, 1011, 64, torch.bfloat16, 1), (100, 1000, 8, torch.float32, 0),
                                                    (520, 600, 256, torch.float32, 1), (1030, 0, 64, torch.bfloat16, 1),
-                                                   (2050, 3, 192, torch.bfloat16, 0), (2079, 0, 256, torch.float32, 1)])
+                                                   (2050, 3, 192, torch.bfloat16, 0), (2079, 0, 256, torch.float32, 1),
+                                                   (520, 960, 256, torch.float32, 1), (2178, 3, 192, torch.bfloat16, 0),
+                                                   (2207, 0, 256, torch.float32, 1)])
 def test_streaming_forms_fused_equal_producers_then_attention(gpu, T, past, rot, wdt, layout):
     c = _prefill_case(T, past, rot, wdt, layout, seed=T + past)
     assert torch.equal(c["cache1"], c["cache2"])
@@ -128,7 +157,8 @@ def test_streaming_forms_fused_equal_producers_then_attention(gpu, T, past, rot,
 
 
 @pytest.mark.parametrize("T,past,rot,wdt,layout", [(521, 1000, 64, torch.bfloat16, 1), (1030, 0, 8, torch.float32, 0),
-                                                   (2049, 3, 256, torch.float32, 1), (2080, 0, 24, torch.bfloat16, 0)])
+                                                   (2049, 3, 256, torch.float32, 1), (2080, 0, 24, torch.bfloat16, 0),
+                                                   (2177, 3, 256, torch.float32, 1), (2208, 0, 24, torch.bfloat16, 0)])
 def test_streaming_forms_fused_non_finite_values(gpu, T, past, rot, wdt, layout):
     # The same call with infinite values in a few tokens (the unfused one is compared with torch above).
     def edit(v):
@@ -143,7 +173,7 @@ def test_streaming_forms_fused_non_finite_values(gpu, T, past, rot, wdt, layout)
 
 
 # Gate and output are accepted at 8-byte alignment, at sizes where each streaming form would take an aligned call.
-@pytest.mark.parametrize("T,past,layout", [(10, 1020, 1), (600, 1020, 0), (1030, 0, 1), (2049, 0, 1)])
+@pytest.mark.parametrize("T,past,layout", [(10, 1020, 1), (600, 1020, 0), (1030, 0, 1), (2200, 0, 1)])
 def test_gate_and_output_at_8_byte_alignment(gpu, T, past, layout):
     out, ref, same = attend(T, past, layout, seed=T, place=shifted)
     assert out.data_ptr() % 16 == 8
@@ -152,11 +182,13 @@ def test_gate_and_output_at_8_byte_alignment(gpu, T, past, layout):
 
 
 # ---- the f32 cache at the model shape (K, V and the probabilities at f32 precision; tiles of 16 keys, a round of 64)
-def f32_cache(T, past, layout, seed, exact_bf16=False, edit=None, place=lambda t: t):
+def f32_cache(T, past, layout, seed, exact_bf16=False, edit=None, place=lambda t: t, query=None):
     g = torch.Generator(device="cuda").manual_seed(seed)
     rnd = lambda *shape: torch.randn(*shape, device="cuda", generator=g)
     n = past + T
     q, gate = rnd(T, HQ, D).bfloat16(), rnd(T, HQ, D).bfloat16()
+    if query is not None:
+        q = query.bfloat16()
     rows = rnd(2, n, HKV, D)
     if exact_bf16:
         rows = rows.bfloat16().float()
@@ -187,6 +219,34 @@ def test_f32_cache_prefill(gpu, T, past, layout, exact_bf16):
     got = from_dev(out)
     # f32 sums of about 1e-6 of the largest product each, then one rounding to bf16 (2^-8 of the value at most)
     assert np.all(np.abs(got - want) <= 2.0 ** -8 * np.abs(want) * 1.001 + 2e-5)
+
+
+@pytest.mark.parametrize("direction", [1, -1])
+@pytest.mark.parametrize("layout,exact_bf16", [(0, True), (1, False), (1, True), (0, False)])
+def test_f32_cache_prefill_rescale(gpu, direction, layout, exact_bf16):
+    # The ramp over seven rounds of 64 keys: each wave's max moves by 12 to 24 log2 units from one of its tiles to its
+    # next.  The values of the ramp that are not exact in bf16 take the products of the middle and low parts.
+    T, past = 100, 333
+    q, k, _ = (torch.from_numpy(x).cuda() for x in score_ramp(T, past, direction))
+
+    def edit(rows):
+        rows[0] = k.bfloat16().float() if exact_bf16 else k
+        rows[0, past:] = rows[0, past:].bfloat16().float()
+
+    out, p, v, gate, _, same = f32_cache(T, past, layout, seed=7, exact_bf16=exact_bf16, edit=edit, query=q)
+    assert same, "appended rows"
+    want = (torch.matmul(p, v).permute(1, 0, 2) * torch.sigmoid(gate)).cpu().numpy()
+    got = from_dev(out)
+    # scores to 80 carry 80 * 2^-23 each in f32 (3 of them: product, scale, maximum), which moves a weight by as much
+    assert np.all(np.abs(got - want) <= (2.0 ** -8 * 1.001 + 3e-5) * np.abs(want) + 5e-5)
+
+
+@pytest.mark.parametrize("T,past,layout,exact_bf16", [(40, 6000, 0, False), (9, 9001, 1, True), (1500, 70, 1, False)])
+def test_f32_cache_prefill_many_rounds(gpu, T, past, layout, exact_bf16):
+    out, p, v, gate, _, same = f32_cache(T, past, layout, seed=T, exact_bf16=exact_bf16)
+    assert same, "appended rows"
+    want = (torch.matmul(p, v).permute(1, 0, 2) * torch.sigmoid(gate)).cpu().numpy()
+    assert np.all(np.abs(from_dev(out) - want) <= 2.0 ** -8 * np.abs(want) * 1.001 + 2e-5)
 
 
 def test_f32_cache_prefill_gate_and_output_at_8_byte_alignment(gpu):
