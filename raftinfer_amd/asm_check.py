@@ -9,8 +9,8 @@ The build therefore scans the kernels' gfx950 assembly and fails on
 * any read of an inline-asm MFMA's destination registers, or (vector registers)
   any write to them, within the MFMA's result latency: a copy of an accumulator
   placed there once computed wrong prefill outputs;
-* any vector instruction that writes an operand of an inline-asm MFMA within
-  the two wait states before it;
+* any vector instruction that writes an operand of an inline-asm MFMA, its
+  accumulator among them, within the two wait states before it;
 * in kernels that address the accumulation registers by number (`owned_agprs`),
   any use of one outside asm: it would overwrite an accumulator.
 """
@@ -39,6 +39,13 @@ def _registers(operand: str):
         else:
             found.append((m.group(4), int(m.group(5), 0), int(m.group(5), 0)))
     return found
+
+
+def _vector_writes(opcode: str, operands):
+    """The registers that a vector instruction writes: its first operand, both of a swap."""
+    if not opcode.startswith("v_"):
+        return []
+    return operands[0] + (operands[1] if "swap" in opcode else [])
 
 
 def _overlap(x, y) -> bool:
@@ -75,7 +82,7 @@ def asm_mfma_hazards(assembly: str, owned_agprs: bool = False) -> list[str]:
         nop = _NOP.match(text)
         if opcode.startswith("v_mfma"):
             if in_asm and operands[0]:
-                for source in operands[1] + operands[2]:
+                for source in operands[1] + operands[2] + operands[3]:
                     for register, left, line in written:
                         if left > 0 and _overlap(register, source):
                             hazards.append(f"line {number}: '{text}' reads a register written at line {line}, "
@@ -84,7 +91,7 @@ def asm_mfma_hazards(assembly: str, owned_agprs: bool = False) -> list[str]:
         elif nop is None:
             stores = opcode.startswith("ds_write") or "store" in opcode
             reads = [r for x in (operands if stores else operands[1:]) for r in x]
-            writes = [r for r in operands[0] if r[0] == "v"] if opcode.startswith("v_") else []
+            writes = [r for r in _vector_writes(opcode, operands) if r[0] == "v" and r not in reads]
             for verb, registers in (("reads", reads), ("writes", writes)):
                 for register in registers:
                     for dest, left, line in pending:
@@ -101,6 +108,6 @@ def asm_mfma_hazards(assembly: str, owned_agprs: bool = False) -> list[str]:
         if issued is not None:
             pending.append([issued, RESULT_WAIT_STATES, number])
         written = [e for e in written if e[1] > 0]
-        if opcode.startswith("v_") and not opcode.startswith("v_mfma") and operands[0]:
-            written.append([operands[0][0], OPERAND_WAIT_STATES, number])
+        if not opcode.startswith("v_mfma"):
+            written += [[r, OPERAND_WAIT_STATES, number] for r in _vector_writes(opcode, operands)]
     return hazards

@@ -51,6 +51,14 @@ def test_vector_results_operand_writes_and_owned_registers():
     write = "\tv_add_f32_e32 v32, v1, v2\n"
     assert len(asm_mfma_hazards(write + "\ts_nop 0\n" + mfma)) == 1
     assert asm_mfma_hazards(write + "\ts_nop 1\n" + mfma) == []
+    # ... also the accumulator that goes in, and both registers of a swap
+    for line in ("\tv_accvgpr_write_b32 a20, v9\n", "\tv_permlane32_swap_b32_e32 v1, v31\n",
+                 "\tv_permlane32_swap_b32_e32 v9, v1\n", "\tv_swap_b32 v1, v7\n"):
+        agpr = MFMA.replace("\ts_nop 1\n", "")
+        assert len(asm_mfma_hazards(line + agpr)) == 1, line
+        assert asm_mfma_hazards(line + "\ts_nop 1\n" + agpr) == [], line
+    for line in ("\tv_permlane32_swap_b32_e32 v1, v41\n", "\tv_permlane16_swap_b32_e32 v41, v1\n"):
+        assert len(asm_mfma_hazards(mfma + line)) == 1, line
     # registers named in hexadecimal, and the rule for kernels that own the accumulation registers
     assert len(asm_mfma_hazards(MFMA.replace("a[16:31]", "a[0x80:0x8f]") + "\tv_accvgpr_read_b32 v0, a[0x81]\n")) == 1
     spill = "\tv_accvgpr_write_b32 a3, v9\n"
