@@ -217,7 +217,10 @@ int raftinfer_amd_online_attention_decode_static_workspace(
     raftinfer_amd_decode_plan plan, const uint32_t *device_position, void *stream);
 /* Measurement entry points (no reference counterpart): validate like the
  * calls above, then enqueue only the dominant kernel (the split-K partition
- * kernel; the prefill attention kernel without the K/V append). */
+ * kernel; the prefill attention kernel without the K/V append).  The partition
+ * kernel for bf16 activations on a bf16 cache forms the append itself; on an f32
+ * cache or for f32 activations nothing is appended and the cache must hold the
+ * new token's row. */
 int raftinfer_amd_online_attention_decode_partition_only(
     const void *query, const void *key, const void *value, const void *gate, void *output,
     void *kv_cache, size_t kv_cache_bytes, void *workspace, size_t workspace_bytes,

@@ -160,7 +160,9 @@ void qwen35_online_attention_decode_static_workspace(
 // exactly like qwen35_online_attention_decode / _prefill, then enqueue only the
 // dominant kernel -- the split-K partition kernel of a split plan, or the
 // prefill attention kernel without the K/V append -- so a benchmark can time
-// it alone with events on the same stream.
+// it alone with events on the same stream.  The partition kernel for bf16
+// activations on a bf16 cache forms the append itself; on an f32 cache or for
+// f32 activations nothing is appended and the cache must hold the new token's row.
 void qwen35_online_attention_decode_partition_only(
     const void *query, const void *key, const void *value, const void *gate, void *output,
     void *kv_cache, std::size_t kv_cache_bytes, void *workspace, std::size_t workspace_bytes,

@@ -892,48 +892,48 @@ void launch_decode(const void *query, const void *key, const void *value, const 
     launch_decode_mfma<false>(args, g, kHeadDim, out, workspace, shape, plan, ws, device_position,
                               stream, partition_only, FusedNormRope{});
   } else {
-  const bool single = plan.resolved_mode == Qwen35DecodeAttentionMode::single_block;
-  if (partition_only) require<Err>(plan.partition_tokens != 0, "partition-only decode needs a split-K plan");
-  const ScanArgs<ActT, CacheT> args{q, static_cast<const ActT *>(key), static_cast<const ActT *>(value), cache,
-                                    shape.max_context_tokens, head_major};
-  const unsigned single_grid = xcd_grid<kScanSingleDs>(kQueryHeads);
-  const std::size_t host_ctx = shape.past_tokens + 1;
-  if (single || (device_position == nullptr && !partition_only && host_ctx < plan.split_k_threshold_tokens)) {
-    decode_scan_single_kernel<ActT, CacheT><<<single_grid, kScanWaves * 64, 0, stream>>>(
-        args, g, out, shape.past_tokens, device_position);
-    check_launch<Err>("qwen35_online_attention_decode_gfx950_hd256");
-    return;
-  }
-  const std::size_t max_partitions = ceil_div(shape.max_context_tokens, plan.partition_tokens,
-                                              "online decode maximum partition capacity overflow");
-  const std::size_t units = checked_mul<Err>(kKvHeads, plan.active_partition_capacity,
-                                             "online decode partition grid dimension overflow");
-  (void)grid_dim(checked_mul<Err>(units + 8, kSplitDs, "online decode partition grid dimension overflow"),
-                 "online decode partition grid dimension overflow");
-  auto *bytes = static_cast<std::byte *>(workspace);
-  auto *pmax = reinterpret_cast<float *>(bytes + ws.max_offset_bytes);
-  auto *psum = reinterpret_cast<float *>(bytes + ws.sum_offset_bytes);
-  auto *pval = reinterpret_cast<float *>(bytes + ws.value_offset_bytes);
-  // As the bf16 kernels: slice the dims only while the partitions alone leave
-  // the 256 CUs idle.
-  auto go = [&](auto kernel, unsigned split_grid) {
-    kernel<<<split_grid > single_grid ? split_grid : single_grid, kScanWaves * 64, 0, stream>>>(
-        args, g, out, pmax, psum, pval, shape.past_tokens, device_position, plan.active_partition_capacity,
-        max_partitions, plan.partition_tokens, plan.split_k_threshold_tokens, partition_only);
-  };
-  if (units >= 192)
-    go(decode_scan_kernel<ActT, CacheT, 1>, xcd_grid<1>(units));
-  else if (units >= 96)
-    go(decode_scan_kernel<ActT, CacheT, 2>, xcd_grid<2>(units));
-  else
-    go(decode_scan_kernel<ActT, CacheT, kSplitDs>, xcd_grid<kSplitDs>(units));
-  check_launch<Err>(plan.partition_tokens == 256
-                        ? "qwen35_online_attention_decode_split_k_256_partition"
-                        : "qwen35_online_attention_decode_split_k_512_partition");
-  if (partition_only) return;
-  launch_merge<ActT>(g, kHeadDim, out, pmax, psum, pval, shape, plan, max_partitions, device_position,
-                     stream);
-  check_launch<Err>("qwen35_online_attention_decode_split_k_merge");
+    const bool single = plan.resolved_mode == Qwen35DecodeAttentionMode::single_block;
+    if (partition_only) require<Err>(plan.partition_tokens != 0, "partition-only decode needs a split-K plan");
+    const ScanArgs<ActT, CacheT> args{q, static_cast<const ActT *>(key), static_cast<const ActT *>(value), cache,
+                                      shape.max_context_tokens, head_major};
+    const unsigned single_grid = xcd_grid<kScanSingleDs>(kQueryHeads);
+    const std::size_t host_ctx = shape.past_tokens + 1;
+    if (single || (device_position == nullptr && !partition_only && host_ctx < plan.split_k_threshold_tokens)) {
+      decode_scan_single_kernel<ActT, CacheT><<<single_grid, kScanWaves * 64, 0, stream>>>(
+          args, g, out, shape.past_tokens, device_position);
+      check_launch<Err>("qwen35_online_attention_decode_gfx950_hd256");
+      return;
+    }
+    const std::size_t max_partitions = ceil_div(shape.max_context_tokens, plan.partition_tokens,
+                                                "online decode maximum partition capacity overflow");
+    const std::size_t units = checked_mul<Err>(kKvHeads, plan.active_partition_capacity,
+                                               "online decode partition grid dimension overflow");
+    (void)grid_dim(checked_mul<Err>(units + 8, kSplitDs, "online decode partition grid dimension overflow"),
+                   "online decode partition grid dimension overflow");
+    auto *bytes = static_cast<std::byte *>(workspace);
+    auto *pmax = reinterpret_cast<float *>(bytes + ws.max_offset_bytes);
+    auto *psum = reinterpret_cast<float *>(bytes + ws.sum_offset_bytes);
+    auto *pval = reinterpret_cast<float *>(bytes + ws.value_offset_bytes);
+    // As the bf16 kernels: slice the dims only while the partitions alone leave
+    // the 256 CUs idle.
+    auto go = [&](auto kernel, unsigned split_grid) {
+      kernel<<<split_grid > single_grid ? split_grid : single_grid, kScanWaves * 64, 0, stream>>>(
+          args, g, out, pmax, psum, pval, shape.past_tokens, device_position, plan.active_partition_capacity,
+          max_partitions, plan.partition_tokens, plan.split_k_threshold_tokens, partition_only);
+    };
+    if (units >= 192)
+      go(decode_scan_kernel<ActT, CacheT, 1>, xcd_grid<1>(units));
+    else if (units >= 96)
+      go(decode_scan_kernel<ActT, CacheT, 2>, xcd_grid<2>(units));
+    else
+      go(decode_scan_kernel<ActT, CacheT, kSplitDs>, xcd_grid<kSplitDs>(units));
+    check_launch<Err>(plan.partition_tokens == 256
+                          ? "qwen35_online_attention_decode_split_k_256_partition"
+                          : "qwen35_online_attention_decode_split_k_512_partition");
+    if (partition_only) return;
+    launch_merge<ActT>(g, kHeadDim, out, pmax, psum, pval, shape, plan, max_partitions, device_position,
+                       stream);
+    check_launch<Err>("qwen35_online_attention_decode_split_k_merge");
   }
 }
 

@@ -21,9 +21,13 @@
 //   - KS = 4 key groups: each wave streams its own 32-key tiles (no barriers in
 //     the loop); KS = 2: two waves with 64 columns each share a group's tiles,
 //     which halves the bytes and LDS writes per column for one barrier per item.
-//     Barriers and loads bound NB = 1 (128 KiB per round of 4 tiles: 1.4 us),
-//     the card's power NB = 2 (2048 tokens behind 30000: 1.2 PFLOP/s, the rate
-//     that a bf16 matrix product of 8192^3 reaches here).
+//     Counters (share of the wave cycles that the matrix units are busy / that vector
+//     instructions issue / that a wave waits): NB = 1, 512
+//     tokens behind 3584: 32 / 30 / 27%, one chain per SIMD; NB = 2, 2000 tokens: 26 /
+//     35 / 33%, the start, the end and the last workgroups; 6001 tokens: 49 / 34 / 19%
+//     at 2.07 GHz; 2048 behind 30000: 60 / 36 / 16% at 1.70 GHz, where the other kernels
+//     run at 2.3 to 2.4: the card's power bounds the last two (1.0 to 1.2 PFLOP/s, the
+//     rate that a bf16 matrix product of 8192^3 reaches here).
 //   - a masked key has probability 0, and 0 times an infinite or NaN value is not 0:
 //     with NB = 2, a workgroup whose own tokens have such values throws its sums away
 //     and forms them again, the tiles that mask key by key (careful_tile).  With 8
@@ -73,7 +77,11 @@ __device__ __forceinline__ void load_lds_b128_at(const void *base, std::uint32_t
 // The O^T accumulators (2 column blocks x 8 dim blocks x 16 registers) fill the
 // 256 accumulation registers, and are addressed by number from asm: block
 // `kAcc` (8 b + nb) is a[16 kAcc : 16 kAcc + 15].  Left to the register
-// allocator, values of this size were copied and spilled around every tile.
+// allocator, values of this size were copied and spilled around every tile.  What is
+// left of the vector registers does not hold everything with NB = 2: 24 (KS = 4), 33
+// (KS = 2) or 59 (KS = 2 with NormQ) are spilled, none of them inside the loop over
+// whole tiles; two steps of the loop over the last tiles reload 11 to 29, and the wait
+// for a reload also waits for the LDS-direct loads in front of it.
 // acc_fence clobbers the whole file around every tile, so the compiler keeps
 // nothing of its own there (the statements in between carry no clobber list,
 // which took minutes to compile); the build checks that no instruction outside
@@ -151,9 +159,13 @@ template <int NB, int KS> struct Plan {
 // matter at f32 precision are summed in f32.  Cache rows appended from bf16
 // activations have m = l = 0; each half tile is checked, and takes the products
 // with m and l only if some value has more bits.  A tile is 16 keys, so its halves
-// are the same 8 KiB ring items; S and PV are not overlapped.  The vector unit
-// bounds it (the checks and packing of 8192 values per wave and tile).  512 tokens
-// on a token-major f32 cache: 866 us with one wave per row and fp32 FMAs, now 31.
+// are the same 8 KiB ring items; S and PV are not overlapped.  It is a chain at one
+// wave per SIMD: 35 to 39% of the wave cycles issue vector instructions (the checks and
+// packing of 8192 values per wave and tile), 32 to 35% wait, the matrix units are busy
+// for 12 to 16%; with general f32 values 51, 31 and 14%.  512 tokens on a token-major
+// f32 cache: 866 us with one wave per row and fp32 FMAs, now 31 to 33; behind 4000
+// tokens 17,900 us, now 197 where the past is exact in bf16 (rows that bf16 activations
+// appended) and 507 where it is not.
 __device__ __forceinline__ std::uint32_t high_pair(float a, float b) { // truncated bf16 of (a, b)
   return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }

@@ -882,16 +882,13 @@ __device__ __forceinline__ floatx4 mfma4(float a, float b, floatx4 c) {
 constexpr int kLd = kChunkDim + 4; // LDS row stride for 128-wide rows
 constexpr int kLdC = kChunk + 4;   // LDS row stride for 64-wide rows
 
-// Batched staging of a 64 x 128 block of rows (rows >= L repeat row L-1): thread owns
-// rows (tid + 256 r) / 16, dims 8 * ((tid + 256 r) % 16), r = 0..3, so every
-// global load of the block is issued before any of them is consumed.
+// 8 contiguous values as loaded, bf16 ones past the caches.
 template <typename T> struct Chunk8;
 template <> struct Chunk8<bf16_bits> {
   u32x4 w;
   __device__ __forceinline__ void load(const bf16_bits *p) {
     w = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
   }
-  __device__ __forceinline__ void zero() { w = u32x4{0u, 0u, 0u, 0u}; }
   __device__ __forceinline__ float get(int i) const {
     const std::uint32_t x = w[i >> 1];
     return (i & 1) ? bf16_hi(x) : bf16_lo(x);
@@ -903,10 +900,6 @@ template <> struct Chunk8<float> {
     a = reinterpret_cast<const float4 *>(p)[0];
     b = reinterpret_cast<const float4 *>(p)[1];
   }
-  __device__ __forceinline__ void zero() {
-    a = make_float4(0.f, 0.f, 0.f, 0.f);
-    b = a;
-  }
   __device__ __forceinline__ float get(int i) const {
     switch (i) {
     case 0: return a.x; case 1: return a.y; case 2: return a.z; case 3: return a.w;
@@ -915,6 +908,9 @@ template <> struct Chunk8<float> {
   }
 };
 
+// Batched staging of a 64 x 128 block of rows (rows >= L repeat row L-1): thread owns
+// rows (tid + 256 r) / 16, dims 8 * ((tid + 256 r) % 16), r = 0..3, so every
+// global load of the block is issued before any of them is consumed.
 template <typename T> struct RowBlock {
   Chunk8<T> c[4];
   template <typename Addr>
