@@ -626,11 +626,11 @@ __global__ __launch_bounds__(WAVES * 64) void decode_dynamic_mfma_kernel(
 //
 // A single-block step: a workgroup per (query head, one of four dims slices).  The
 // scores bound it, so a workgroup has those of one head: all four heads of a KV head
-// in each of sixteen slices took 8.5 us at 255 tokens and 14.9 at 700 of an f32 cache
-// (now 5.5 and 9.4), and on a bf16 cache 15.5 at 700, more than the 13.4 of one
-// workgroup per head with all dims (now 8.1).  Two tokens per row-group and step on
-// f32 rows, four on bf16 rows: 4000 bf16 tokens 39 -> 32 us, 200 f32 tokens 5.1
-// against 5.6.
+// in each of sixteen slices took 17.0 us at 700 tokens of an f32 cache from memory (now
+// 15.3) and 14.9 at the same cache again and again (9.4), 15.8 and 15.5 on a bf16 cache
+// (11.1 and 8.1; one workgroup per head with all dims 20.7 and 13.4).  Two tokens per
+// row-group and step on f32 rows, four on bf16 rows: 4000 bf16 tokens 39 -> 32 us, 200
+// f32 tokens 5.1 against 5.6.
 constexpr int kScanWaves = 8;
 constexpr int kScanSingleDs = 4;
 template <typename CacheT> constexpr int kScanSingleUnroll = sizeof(CacheT) == 4 ? 2 : 4;
@@ -672,10 +672,12 @@ __device__ __forceinline__ void scan_split_body(unsigned block, const ScanArgs<A
   int dq;
   xcd_unit<DS>(block, unit, dq);
   if (unit >= kKvHeads * capacity) return;
-  // The four KV heads of a partition run side by side where their f32 rows lie side by
-  // side (token-major, 32768 tokens from memory: 69 -> 62 us); rows of one head follow
-  // each other otherwise (head-major f32 67 -> 57 us, bf16 42 -> 39.5).
-  const bool heads_first = DS == 1 && sizeof(CacheT) == 4 && !a.head_major;
+  // The four KV heads of a partition run side by side with up to 64 partitions (16384
+  // tokens from memory, head-major f32: 31.9 us against 33.1, bf16 22.7 against 23.3),
+  // and with more where their f32 rows lie side by side (token-major, 32768 tokens: 62
+  // against 69); else partitions of one head do (head-major f32 67 -> 56, bf16 43.3 ->
+  // 39.4 and 39.6).
+  const bool heads_first = DS == 1 && (capacity <= 64 || (sizeof(CacheT) == 4 && !a.head_major));
   const std::size_t kv_head = heads_first ? unit % kKvHeads : unit / capacity;
   const std::size_t partition = heads_first ? unit / kKvHeads : unit % capacity;
   const std::size_t begin = partition * partition_tokens;

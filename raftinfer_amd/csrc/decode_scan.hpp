@@ -85,13 +85,14 @@ __device__ __forceinline__ void scan_slice(const ScanArgs<ActT, CacheT> &a, std:
   constexpr int kDims = kHeadDim / DS, kPerLane = kDims / 16; // output dims of the slice, of a lane
   constexpr int KW = 16 / sizeof(CacheT), KP = 16 / KW;       // K piece width, pieces per lane
   constexpr int VW = kPerLane < KW ? kPerLane : KW, VP = kPerLane / VW;
-  // Which rows are streamed past the caches.  One dims slice reads a row once; with
-  // both K and V streamed a cache of 134 MB (32768 tokens, one layer over and over)
-  // took 61 us where K alone takes 55, and with neither a cache that has to come from
-  // memory 65 where K alone takes 62.  Slices share K.  Their V rows are their own,
-  // but only two f32 slices gain from streaming (8000 tokens from memory: 23.0 -> 20.5
-  // us; four f32 slices at 3000 tokens 14.3 -> 15.8, bf16 rows 15.3 -> 15.8 at 6000).
-  constexpr bool kStreamK = DS == 1, kStreamV = DS == 2 && sizeof(CacheT) == 4;
+  // Which rows are streamed past the caches: in a split step K where one workgroup
+  // reads it, and V, each slice its own.  From memory (1 GB of caches in turn, us, both
+  // / K alone / neither): f32, 16384 tokens 31.3 / 32.5 / 34.6, 8000 in two slices 22.3
+  // / 23.3, 4096 in four 16.4 / 17.0; bf16, 16384: 23.0 / 23.4 / 24.2.  (One layer over
+  // and over, 268 MB that the memory-side cache half holds, 32768 tokens: 61 / 54 / 55.)
+  // The short rows of a single-block step are better left alone (700 tokens 18.8 with
+  // V streamed, 15.3 without).
+  constexpr bool kSplit = NH == kGroup, kStreamK = kSplit && DS == 1, kStreamV = kSplit;
   // Element of piece p of a lane: 16 KW p + KW r (K), 16 VW p + VW r of the slice (V).
   const CacheT *k_plane = a.cache + cache_row(a.head_major, 0, kv_head, a.max_ctx);
   const CacheT *v_plane = k_plane + a.max_ctx * kKvHeads * kHeadDim + dq * kDims;
