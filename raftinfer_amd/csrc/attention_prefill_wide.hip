@@ -78,10 +78,10 @@ __device__ __forceinline__ void load_lds_b128_at(const void *base, std::uint32_t
 // 256 accumulation registers, and are addressed by number from asm: block
 // `kAcc` (8 b + nb) is a[16 kAcc : 16 kAcc + 15].  Left to the register
 // allocator, values of this size were copied and spilled around every tile.  What is
-// left of the vector registers does not hold everything with NB = 2: 24 (KS = 4), 33
-// (KS = 2) or 59 (KS = 2 with NormQ) are spilled, none of them inside the loop over
-// whole tiles; two steps of the loop over the last tiles reload 11 to 29, and the wait
-// for a reload also waits for the LDS-direct loads in front of it.
+// left of the vector registers does not hold everything with NB = 2: 23 to 28 (KS
+// = 4) or 33 and 34 (KS = 2) are spilled, none of them inside the loop over whole
+// tiles; two steps of the loop over the last tiles have 16 to 19 scratch accesses, and
+// the wait for a reload also waits for the LDS-direct loads in front of it.
 // acc_fence clobbers the whole file around every tile, so the compiler keeps
 // nothing of its own there (the statements in between carry no clobber list,
 // which took minutes to compile); the build checks that no instruction outside
@@ -195,11 +195,26 @@ template <bool F32> using CacheElem = std::conditional_t<F32, float, bf16_bits>;
 // everything anew and is not the streaming loop run again: values kept for either
 // took registers in the streaming loop and its ends (6001 tokens of finite values:
 // 308 us, 313 to 318 with a second run of the loop, 449 with the Q operands kept).
+// Its arguments are the kernel's, loaded again for the same reason: kept in scalar
+// registers they were spilled (fused, 1500 tokens behind 2000: 115.5 us in place of
+// 107.2).
+struct WideArguments { // as the kernel argument segment holds those of prefill_wide_kernel
+  const bf16_bits *query, *key_in, *value_in, *gate;
+  bf16_bits *output;
+  const bf16_bits *cache;
+  std::size_t tokens, max_ctx, past;
+  PrefillNormRope nq;
+};
 template <int kTok, bool HeadMajor, bool FromInput, bool NormQ>
-__device__ __forceinline__ void careful_tile(const bf16_bits *query, const bf16_bits *key_in, const bf16_bits *value_in,
-                                             const bf16_bits *gate, bf16_bits *output, const bf16_bits *cache,
-                                             std::size_t tokens, std::size_t max_ctx, std::size_t past,
-                                             const PrefillNormRope &nq, unsigned lds0) {
+__device__ __forceinline__ void careful_tile(unsigned lds0) {
+  auto arguments = reinterpret_cast<std::uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr());
+  asm volatile("" : "+s"(arguments));
+  const auto &args = *(const __attribute__((address_space(4))) WideArguments *)arguments;
+  const bf16_bits *query = args.query, *key_in = args.key_in, *value_in = args.value_in, *gate = args.gate;
+  const bf16_bits *cache = args.cache;
+  bf16_bits *output = args.output;
+  const std::size_t tokens = args.tokens, max_ctx = args.max_ctx, past = args.past;
+  const PrefillNormRope nq{args.nq.weight, args.nq.weight_f32, args.nq.pairs, args.nq.ratio, args.nq.epsilon};
   int tid = threadIdx.x;
   unsigned block = blockIdx.x;
   asm volatile("" : "+v"(tid), "+s"(block)); // (nothing of this is formed before the streaming loop)
@@ -407,10 +422,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   };
 
   // The lane index again: what is derived from it is not computed before the tile
-  // loop and kept (or spilled) over it.
+  // loop and kept (or spilled) over it.  With NB = 2 the index is counted anew as well:
+  // kept in a register, it had the tail of the loop spill 55 in place of 34 (KS = 2,
+  // NormQ: 2500 tokens 100 us in place of 92; without NormQ, 600 behind 800: 36.5 in
+  // place of 35.6).  With KS = 4 and NormQ it is better kept (1500: 56.8 against 59.3).
   auto late_lane = [&]() __attribute__((always_inline)) {
-    int l = threadIdx.x & 63;
-    asm volatile("" : "+v"(l));
+    int l;
+    if constexpr (NB == 2 && (kShare > 1 || !NormQ)) {
+      asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+    } else {
+      l = threadIdx.x & 63;
+      asm volatile("" : "+v"(l));
+    }
     return l;
   };
   // ---- staging: ring items of 8 loads (1 KiB) per wave.
@@ -1274,8 +1297,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
   if constexpr (kWatch) {
     if (!again) return;
     __syncthreads(); // the flags have been read
-    careful_tile<kTok, HeadMajor, FromInput, NormQ>(query, key_in, value_in, gate, output, cache, tokens, max_ctx, past, nq,
-                                                    lds0);
+    careful_tile<kTok, HeadMajor, FromInput, NormQ>(lds0);
   }
 }
 
