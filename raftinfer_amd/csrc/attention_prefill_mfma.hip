@@ -544,25 +544,29 @@ __global__ __launch_bounds__(kThreads) void prefill_mfma_kernel(
 // tokens), and below them where the longer start and end of the streaming
 // kernel is made up for.  Measured (us; short8 / stream8 / stream16 / stream32,
 // tokens behind past keys):
-//   to 512, line at 1024 keys: 64 behind 600: 17.0 / 18.5 / 28, behind 1024: 21.7 /
-//     19.9 / 30 / 45; 512 behind 0: 12.9 / 15.4 / 21 / 30, behind 400: 21.9 / 22.6 /
+//   to 512, line at 1024 keys: 64 behind 600: 17.0 / 18.5 / 28, behind 1024: 21.6 /
+//     19.8 / 30 / 45; 512 behind 0: 12.9 / 15.4 / 21 / 30, behind 400: 21.9 / 22.6 /
 //     32, behind 512: 22.2 / 22.7, behind 513: 23.2 / 22.6 / 33, behind 1000: 28.0 /
 //     27.2 / 39
-//   to 1024, line at 1440: 513 behind 800: 34.7 / 33.9 / 35.7, behind 1000: 39.2 /
-//     38.5 / 38.7; 600 behind 513: 30.9 / 32.5 / 33.8, behind 1000: 41.6 / 41.1 /
-//     39.2; 900 behind 513: 40.4 / 41.4 / 41.8, behind 600: 42.1 / 41.7 / 41.6;
-//     1024 behind 513: 44.2 / 44.4 / 42.8, behind 4000: 125 / 113 / 94
-//   1024: 1025 behind 0: 29.5 / 31.4 / 29.5 / 45, 1100 behind 0: 32.1 / 33.7 / 29.9
-//   2048 and 2176: 2048 behind 0: 70 / 71 / 59.1 / 69.1, behind 2000: 171 / 157 /
-//     126.8 / 129.4; 2049 behind 0 (its 260 workgroups of 32 begin a second pass,
-//     as the 516 of 16 do): 75 / 75 / 68.2 / 69.1, behind 1000: 139 / 130 / 120 /
-//     110; 2176 behind 0: 80 / 80 / 68.7 / 71.0, 2240: 84 / 84 / 77.1 / 74.0
-//   beyond: 4096 behind 0: 228 / 218 / 172 / 148, 2304 behind 4000: 325 / 286 / 247 /
-//     256, 2500 behind 4000: 338 / 300 / 258 / 262.
+//   to 1024, line at 1344 keys, above 832 tokens (more than 208 of the 256 CUs) at 1440:
+//     513 behind 700: 33.2 / 34.2 / 35.3, behind 831: 36.2 / 34.6 / 35.1, behind 900:
+//     37.8 / 38.3 / 37.9, behind 1000: 39.5 / 38.6 / 38.3; 600 behind 600: 32.6 / 35.0 / 36.0, behind
+//     800: 37.3 / 36.7 / 36.2; 900 behind 400: 37.8 / 39.8 / 38.2, behind 450: 39.3 /
+//     40.0 / 38.4, behind 513: 40.6 / 41.3 / 41.2, behind 600: 42.3 / 41.9 / 41.1; 1024
+//     behind 300: 38.7 / 40.6 / 39.6, behind 450: 42.9 / 42.9 / 42.2, behind 2000: 79 /
+//     71 / 65 / 93
+//   1024: 1025 behind 0: 29.4 / 31.4 / 28.8 / 45, 1100 behind 0: 32.1 / 33.7 / 29.6
+//   2048 and 2176: 2048 behind 0: 70 / 73 / 59.5 / 69, behind 2000: 171 / 157 / 124.5 /
+//     127.7; 2049 behind 0 (its 260 workgroups of 32 begin a second pass, as the 516 of
+//     16 do): 76 / 77 / 66.7 / 68.8, behind 1000: 139 / 130 / 120 / 110; 2176 behind 0:
+//     80 / 81 / 68.4 / 70.4, 2240: 84 / 85 / 75.9 / 73.2
+//   beyond: 4096 behind 0: 231 / 220 / 171 / 148, 2304 behind 4000: 323 / 284 / 246 /
+//     254, 2500 behind 4000: 339 / 296 / 256 / 260.
 PrefillForm prefill_plan(std::size_t tokens, std::size_t past) {
   if (tokens > 2048 && past + tokens > 2176) return PrefillForm::stream32;
   if (tokens > 1024) return PrefillForm::stream16;
-  if (tokens > 512) return past + tokens >= 1440 ? PrefillForm::stream16 : PrefillForm::short8;
+  if (tokens > 512)
+    return past + tokens >= (tokens > 832 ? 1440u : 1344u) ? PrefillForm::stream16 : PrefillForm::short8;
   return past + tokens > 1024 ? PrefillForm::stream8 : PrefillForm::short8;
 }
 

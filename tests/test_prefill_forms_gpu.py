@@ -55,8 +55,9 @@ def attend(T, past, layout, seed, edit=None, place=lambda t: t, edit_all=None):
 # query tile and of a key tile, an odd and an even number of key tiles.
 @pytest.mark.parametrize("T,past", [(2, 1022), (7, 1050), (33, 1000), (511, 513), (512, 512), (513, 513), (577, 1055),
                                     (1025, 0), (1039, 0), (1040, 65), (1072, 31), (2049, 0), (2080, 0), (2081, 40),
-                                    (2113, 7), (2, 1023), (512, 513), (513, 926), (513, 927), (577, 863), (1024, 416), (2176, 0), (2049, 128),
-                                    (2177, 0), (2208, 0), (2209, 40), (2241, 7)])
+                                    (2113, 7), (2, 1023), (512, 513), (513, 830), (513, 831), (577, 863), (833, 510),
+                                    (833, 607), (1024, 416), (2176, 0), (2049, 128), (2177, 0), (2208, 0), (2209, 40),
+                                    (2241, 7)])
 @pytest.mark.parametrize("layout", [0, 1])
 def test_streaming_forms_against_torch(gpu, T, past, layout):
     out, ref, same = attend(T, past, layout, seed=T + past)
