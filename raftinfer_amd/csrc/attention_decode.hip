@@ -619,7 +619,7 @@ __global__ __launch_bounds__(WAVES * 64) void decode_dynamic_mfma_kernel(
 // computing the scores of all its keys and reading its own part of V.  With the whole
 // 256 dims in one workgroup a context of 3000 tokens had 48 workgroups, and a step was
 // four launches (append, early exit of the single-block kernel, partitions, merge):
-// 26.6 us on an f32 token-major cache, 15 of them the partitions.  Sliced, with the
+// 26.8 us on an f32 token-major cache, 15 of them the partitions.  Sliced, with the
 // append and the choice of path inside, it is two launches and 15.9 us, 11.4 to 12.5
 // of them the partitions: with four slices they read 61 MB (K four times, V once; 25
 // MB are the cache's own) and repeat the scores four times on the vector units.

@@ -550,8 +550,8 @@ __global__ __launch_bounds__(kThreads) void prefill_mfma_kernel(
 //     27.2 / 39
 //   to 1024, line at 1344 keys, above 832 tokens (more than 208 of the 256 CUs) at 1440:
 //     513 behind 700: 33.2 / 34.2 / 35.3, behind 831: 36.2 / 34.6 / 35.1, behind 900:
-//     37.8 / 38.3 / 37.9, behind 1000: 39.5 / 38.6 / 38.3; 600 behind 600: 32.6 / 35.0 / 36.0, behind
-//     800: 37.3 / 36.7 / 36.2; 900 behind 400: 37.8 / 39.8 / 38.2, behind 450: 39.3 /
+//     37.8 / 38.3 / 37.9, behind 1000: 39.5 / 38.6 / 38.3; 600 behind 600: 32.6 / 35.0 /
+//     36.0, behind 800: 37.3 / 36.7 / 36.2; 900 behind 400: 37.8 / 39.8 / 38.2, behind 450: 39.3 /
 //     40.0 / 38.4, behind 513: 40.6 / 41.3 / 41.2, behind 600: 42.3 / 41.9 / 41.1; 1024
 //     behind 300: 38.7 / 40.6 / 39.6, behind 450: 42.9 / 42.9 / 42.2, behind 2000: 79 /
 //     71 / 65 / 93

@@ -205,6 +205,7 @@ struct WideArguments { // as the kernel argument segment holds those of prefill_
   std::size_t tokens, max_ctx, past;
   PrefillNormRope nq;
 };
+static_assert(sizeof(WideArguments) == 104, "the arguments lie without padding in between");
 template <int kTok, bool HeadMajor, bool FromInput, bool NormQ>
 __device__ __forceinline__ void careful_tile(unsigned lds0) {
   auto arguments = reinterpret_cast<std::uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr());
