@@ -50,9 +50,10 @@ def attend(T, past, layout, seed, edit=None, place=lambda t: t, edit_all=None):
     return out, ref, torch.equal(written, full)
 
 
-# 8 tokens per workgroup: a single ragged query tile, one key tile more or less than a round of four, the first
-# contexts that take the form; 16: its first prompt with and without a past; 32: prompts that end in every part of a
-# query tile and of a key tile, an odd and an even number of key tiles.
+# Both sides of every line of prefill_plan.  8 tokens per workgroup: a single ragged query tile, one key tile more or less
+# than a round of four, the first contexts that take the form; 16: its first prompt with and without a past, its last
+# (2176 keys), query and key tiles of every length, behind a past from 1344 and 1440 keys; 32 (from 2177 keys): prompts
+# that end in every part of a query tile and of a key tile, an odd and an even number of key tiles.
 @pytest.mark.parametrize("T,past", [(2, 1022), (7, 1050), (33, 1000), (511, 513), (512, 512), (513, 513), (577, 1055),
                                     (1025, 0), (1039, 0), (1040, 65), (1072, 31), (2049, 0), (2080, 0), (2081, 40),
                                     (2113, 7), (2, 1023), (512, 513), (513, 830), (513, 831), (577, 863), (833, 510),
